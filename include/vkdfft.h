@@ -157,6 +157,9 @@ int vkx_plan_exec_timed(uint64_t plan, const uint64_t* bufs, int num_bufs, const
 int vkx_twiddles(uint64_t dst, int n, const int* radices, int num_passes, int double_precision, uint64_t stream);
 /* Roots of unity r[k] = exp(-2 pi i k / n), k in [0, n) (real-FFT pre/post-processing). */
 int vkx_roots(uint64_t dst, int n, int double_precision, uint64_t stream);
+/* Twiddles between the passes of a split transform: dst[r * cols + c] = exp(-2 pi i r c step / n),
+ * r < rows, c < cols, the phase reduced mod n in exact integers. */
+int vkx_outer_roots(uint64_t dst, int rows, int cols, int step, int n, int double_precision, uint64_t stream);
 /* dst[i] = sum over b < batch of src[b*count + i] for float (or double) arrays, summed
  * in a fixed order (deterministic).  No counterpart in the reference: used by the
  * hand-written convolution adjoint to reduce the kernel gradient over the batch. */

@@ -315,3 +315,43 @@ def test_graph_replay_after_another_plan_needs_more_scratch():
         g.submit()
         vd.synchronize()
         _check(sizes, parts, dst.read(0))
+
+
+@pytest.mark.parametrize("n,count", [(16384 * 2, 3), (59049, 1), (463050, 2), (864360, 1), (823543, 2), (1 << 21, 1),
+                                     (11 ** 3 * 13, 5), (1 << 20, 9)])
+def test_two_launch_transforms(n, count):
+    """Tiles that do not divide (59049 = 243^2 and others), three and four passes, tiles of
+    four, and a batch of several chunks (9 x 2^20): forward and back.  FP32 Stockham error
+    grows with the square root of the passes; 1e-6 is twice what eight passes give."""
+    rng = np.random.default_rng(n % 1000)
+    x = (rng.standard_normal((count, n)) + 1j * rng.standard_normal((count, n))).astype(np.complex64)
+    buf = vd.asbuffer(x)
+    vd.fft.fft(buf)
+    assert O.rel_l2(buf.read(0), np.fft.fft(x.astype(np.complex128), axis=1)) < 1e-6
+    vd.fft.ifft(buf)
+    assert O.rel_l2(buf.read(0), x) < 2e-6
+
+
+def test_two_launch_transform_in_a_graph():
+    """Recorded, replayed several times with eager work between, and on another stream."""
+    n = 1 << 17
+    rng = np.random.default_rng(1)
+    x = (rng.standard_normal((2, n)) + 1j * rng.standard_normal((2, n))).astype(np.complex64)
+    ref = np.fft.fft(x.astype(np.complex128), axis=1)
+    buf, other = vd.asbuffer(x), vd.asbuffer(x)
+    g = vd.CommandGraph()
+    vd.fft.fft(buf, graph=g)
+    for _ in range(3):
+        buf.write(x)
+        g.submit()
+        other.write(x)
+        vd.fft.fft(other)
+        vd.synchronize()
+        assert O.rel_l2(buf.read(0), ref) < 1e-6 and O.rel_l2(other.read(0), ref) < 1e-6
+    import torch
+    s = torch.cuda.Stream()
+    other.write(x)
+    with vd.stream_scope(s):
+        vd.fft.fft(other)
+        vd.synchronize()
+    assert O.rel_l2(other.read(0), ref) < 1e-6

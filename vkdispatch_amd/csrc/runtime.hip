@@ -95,6 +95,19 @@ __global__ void roots_kernel(T* out, int n) {
   out[2 * k + 1] = (T)s;
 }
 
+// out[r][c] = exp(-2 pi i r c step / n), r c step reduced mod n in integers
+template <typename T>
+__global__ void outer_roots_kernel(T* out, int rows, int cols, int step, int n) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)rows * cols) return;
+  const unsigned long long r = (unsigned long long)(i / cols), c = (unsigned long long)(i % cols);
+  const unsigned long long m = (r * c % (unsigned long long)n) * (unsigned long long)step % (unsigned long long)n;
+  double s, co;
+  sincospi(-2.0 * (double)m / (double)n, &s, &co);
+  out[2 * i] = (T)co;
+  out[2 * i + 1] = (T)s;
+}
+
 // dst[i] = sum_b src[b * count + i] (fixed summation order: deterministic)
 template <typename T>
 __global__ void batch_sum_kernel(T* __restrict__ dst, const T* __restrict__ src, int batch, long long count) {
@@ -454,6 +467,23 @@ int vkx_roots(uint64_t dst, int n, int double_precision, uint64_t stream) {
   else
     hipLaunchKernelGGL(roots_kernel<float>, dim3(blocks), dim3(threads), 0, S(stream),
                        reinterpret_cast<float*>(dst), n);
+  VKX_HIP(hipGetLastError());
+  return 0;
+}
+
+int vkx_outer_roots(uint64_t dst, int rows, int cols, int step, int n, int double_precision, uint64_t stream) {
+  if (!dst) return fail("vkx_outer_roots", "null destination");
+  if (n < 1 || rows < 1 || cols < 1 || step < 1) return fail("vkx_outer_roots", "bad size");
+  const long long count = (long long)rows * cols;
+  const int threads = 256;
+  const long long blocks = (count + threads - 1) / threads;
+  if (blocks > 0x7fffffffll) return fail("vkx_outer_roots", "table too large");
+  if (double_precision)
+    hipLaunchKernelGGL(outer_roots_kernel<double>, dim3((unsigned)blocks), dim3(threads), 0, S(stream),
+                       reinterpret_cast<double*>(dst), rows, cols, step, n);
+  else
+    hipLaunchKernelGGL(outer_roots_kernel<float>, dim3((unsigned)blocks), dim3(threads), 0, S(stream),
+                       reinterpret_cast<float*>(dst), rows, cols, step, n);
   VKX_HIP(hipGetLastError());
   return 0;
 }

@@ -22,6 +22,7 @@ from ..buffer import Buffer, RFFTBuffer
 from ..graph import CommandGraph, dispatch
 from ..shader_map import MappingFunction
 from . import precision as prec
+from .kernels import SpillError
 from .shader_factories import (get_transposed_size, make_convolution_shader, make_fft_shader,
                                make_transpose_shader, register_plan_cache)
 
@@ -133,15 +134,15 @@ def fft(*buffers: Buffer, buffer_shape: Tuple = None, graph: CommandGraph = None
 def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2c, input_map, output_map, out_t,
                              comp_t, signal_range, graph) -> bool:
     """Lengths outside the single-workgroup kernels (a prime factor above 31, or more
-    than 16384 points) run on the ragged executor (mixed radix through global scratch,
-    Bluestein for large primes): contiguous axis, complex64, no hooks, in place."""
+    than 16384 points): contiguous axis, complex64, no hooks, in place.  Lengths that
+    split run as two launches compiled for them (fft/long.py), the others on the ragged
+    executor (mixed radix through global scratch, Bluestein for large primes)."""
     from .planner import AxisGeometry
     geom = AxisGeometry.of(tuple(buffer_shape), axis)
     if (geom.S != 1 or r2c or input_map is not None or output_map is not None or signal_range is not None
             or out_t is not dt.complex64 or comp_t not in (dt.complex64, dt.complex32)):
         return False
-    from .ragged import RaggedFFT
-    plan = _uniform_ragged(geom.N, geom.OUTER, bool(inverse), bool(normalize))
+    plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize))
     buf = buffers[0]
     if graph is not None:
         graph.record_callable(plan.bind(buf))
@@ -150,21 +151,36 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
     return True
 
 
-def _uniform_ragged(n, count, inverse, normalize):
+def _uniform_plan(n, count, inverse, normalize):
+    from . import long
     from .ragged import RaggedFFT
     key = (n, count, inverse, normalize)
-    if key not in _UNIFORM_RAGGED:
+    if key not in _UNIFORM_PLANS:
+        if long.split_length(n) is not None:
+            try:
+                _UNIFORM_PLANS[key] = long.LongFFT(n, count, inverse, normalize)
+                return _UNIFORM_PLANS[key]
+            except SpillError:  # a radix list whose kernel does not fit the registers
+                pass
         plan = RaggedFFT([n] * count, inverse=inverse, normalize=normalize, block=512)
         if plan.n_items > count and count > 128:
             # many tiled transforms: 256-thread workgroups (65536 x 256 points: 298 vs
             # 371 us); whole transforms and small tiled batches run faster at 512
             plan.block = plan.block_first = 256
-        _UNIFORM_RAGGED[key] = plan
-    return _UNIFORM_RAGGED[key]
+        _UNIFORM_PLANS[key] = plan
+    return _UNIFORM_PLANS[key]
 
 
-_UNIFORM_RAGGED: dict = {}
-register_plan_cache(_UNIFORM_RAGGED.clear)
+_UNIFORM_PLANS: dict = {}
+
+
+def _clear_uniform_plans() -> None:
+    from . import long
+    _UNIFORM_PLANS.clear()
+    long.clear()
+
+
+register_plan_cache(_clear_uniform_plans)
 
 
 def fft2(buffer: Buffer, graph: CommandGraph = None, print_shader: bool = False, input_map: MappingFunction = None,

@@ -99,6 +99,7 @@ _SIGS = {
     "vkx_twiddles": ([_U64, ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.c_int, ctypes.c_int, _U64],
                      ctypes.c_int),
     "vkx_roots": ([_U64, ctypes.c_int, ctypes.c_int, _U64], ctypes.c_int),
+    "vkx_outer_roots": ([_U64] + [ctypes.c_int] * 5 + [_U64], ctypes.c_int),
     "vkx_batch_sum": ([_U64, _U64, ctypes.c_int, ctypes.c_longlong, ctypes.c_int, _U64], ctypes.c_int),
     "vkx_chirp": ([_U64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _U64], ctypes.c_int),
     "vkx_ragged_exec": ([_U64, ctypes.c_int, _U64, ctypes.c_int, _U64, ctypes.c_longlong, ctypes.c_int, ctypes.c_int,
