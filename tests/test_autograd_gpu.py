@@ -105,3 +105,32 @@ def test_differentiable_convolution_32x1024x1024():
     assert O.rel_l2(y.detach().double().cpu().numpy(), y64.detach().cpu().numpy()) < 1e-5
     assert O.rel_l2(xa.grad.double().cpu().numpy(), x64.grad.cpu().numpy()) < 1e-5
     assert O.rel_l2(ka.grad.double().cpu().numpy(), k64.grad.cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("shape,dtype", [((3, 64, 48), torch.float32), ((5, 210, 130), torch.float32), ((1, 32, 2), torch.float32),
+                                         ((33, 128, 66), torch.float32), ((2, 1024, 34), torch.float32),
+                                         ((2, 31, 30), torch.float32), ((9, 96, 1000), torch.float32),
+                                         ((3, 64, 48), torch.float64), ((2, 512, 36), torch.float64)])
+@pytest.mark.parametrize("which", ["both", "x", "k"])
+def test_packed_columns_and_their_adjoint(shape, dtype, which):
+    """Columns that do not fill a tile (24, 65, 33, 17 of them), one column only, one image,
+    groups that end early (33 images), a height without a column tile (31): output and
+    gradients against torch.fft in FP64.  FP32 bound: six FFT passes at 3e-7 and a sum."""
+    g = torch.Generator().manual_seed(shape[1])
+    x, gy = (torch.randn(shape, generator=g, dtype=torch.float64) for _ in range(2))
+    k = torch.randn(shape[1:], generator=g, dtype=torch.float64)
+    F = torch.fft
+    X, K, G = F.rfft2(x.to(dtype).double()), F.rfft2(k.to(dtype).double()), F.rfft2(gy.to(dtype).double())
+    want = {"y": F.irfft2(X * K.conj(), s=shape[1:]), "x": F.irfft2(G * K, s=shape[1:]),
+            "k": F.irfft2((X * G.conj()).sum(0), s=shape[1:])}
+    xd = x.to(dtype).cuda().requires_grad_(which != "k")
+    kd = k.to(dtype).cuda().requires_grad_(which != "x")
+    y = _fft_conv()(xd, kd)
+    y.backward(gy.to(dtype).cuda())
+    tol = 2e-6 if dtype is torch.float32 else 1e-13
+    for name, got in (("y", y.detach()), ("x", xd.grad), ("k", kd.grad)):
+        if got is None:
+            assert which != "both" and name not in ("y", which)
+            continue
+        ref = want[name]
+        assert float((got.cpu().double() - ref).norm() / ref.norm()) < tol, name

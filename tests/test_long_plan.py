@@ -27,7 +27,7 @@ def test_tiles_stay_in_bounds(n):
             assert max(slots(m, r, t.TT) for r in t.radices) <= LG.MAX_RADIX
             # LDS positions (b, pos): all different, all inside (vkx_long.h tile_addr)
             pos, b = np.arange(m)[:, None], np.arange(t.B)[None, :]
-            addr = pos * t.pitch + b + (pos >> t.lsh) * t.B
+            addr = pos * t.pitch + b + pos // t.radices[0] * t.B
             assert len(np.unique(addr)) == m * t.B and addr.max() < t.lds_elems
 
 

@@ -819,6 +819,10 @@ __device__ __forceinline__ void conv_body(const KParams& prm) {
 //          (imaginary parts of X[0] and X[M] do not contribute, as in a
 //           complex inverse followed by taking the real part)
 // ---------------------------------------------------------------------------
+// C::PACKED (optional): a row's spectrum is M values, X[0] + i X[M] (both real) in slot 0.
+template <class C, class = void> struct packed_of { static constexpr bool value = false; };
+template <class C> struct packed_of<C, decltype((void)C::PACKED)> { static constexpr bool value = C::PACKED; };
+
 // OOP = true: real rows are read from slot 1 (pitch C::IN_OS reals) and the
 // spectrum written to slot 0; otherwise the RFFTBuffer in slot 0 is used in place.
 template <class C, class S, bool OOP = false>
@@ -869,8 +873,12 @@ __device__ __forceinline__ void rfft_body(const KParams& prm) {
       const cpx<real> d{zk.x - zm.x, zk.y + zm.y};
       const cpx<real> o{h * d.y, -h * d.x};
       const cpx<real> t = cmul(roots[k], o);
-      xout[ob + (u32)k] = ccvt<S>(e + t);
-      xout[ob + (u32)(M - k)] = ccvt<S>(conj(e - t));
+      if (packed_of<C>::value && k == 0) {
+        xout[ob] = ccvt<S>(cpx<real>{e.x + t.x, e.x - t.x});
+      } else {
+        xout[ob + (u32)k] = ccvt<S>(e + t);
+        xout[ob + (u32)(M - k)] = ccvt<S>(conj(e - t));
+      }
     }
   }
 }
@@ -898,7 +906,8 @@ __device__ __forceinline__ void irfft_body(const KParams& prm) {
     const u32 ib = g.outer * C::IN_OS;
     for_layout<C, F0::R>(g.t, [&](auto slot, u32 n) {
       cpx<real> a = ccvt<real>(Xin[ib + n]);
-      cpx<real> bm = ccvt<real>(Xin[ib + (u32)M - n]);
+      cpx<real> bm = ccvt<real>(Xin[ib + (packed_of<C>::value && n == 0u ? 0u : (u32)M - n)]);
+      if (packed_of<C>::value && n == 0u) bm.x = a.y;
       if (n == 0u) { a.y = (real)0; bm.y = (real)0; }
       const cpx<real> e{a.x + bm.x, a.y - bm.y};
       const cpx<real> d{a.x - bm.x, a.y + bm.y};

@@ -16,49 +16,76 @@
 
 namespace vkx {
 
-// LDS element (b, pos) of a tile at pitch C::PITCH per position; every 2^C::LSH
-// positions the banks are moved on by C::B, so that the first exchange, in which
-// neighbouring threads write a radix apart, does not meet the same banks.
+// LDS element (b, pos) of a tile at pos PITCH + b, plus B for every R0 positions (R0: the
+// first radix): in the first exchange neighbouring threads write R0 positions apart and
+// would meet the same banks.  Every later stride is a multiple of R0, so a butterfly's
+// legs are constant offsets from one address.
+template <class C> struct tile_first { static constexpr int value = pl_first<typename C::fwd>::type::R; };
 template <class C> __device__ __forceinline__ int tile_addr(int b, int pos) {
-  return pos * C::PITCH + b + (pos >> C::LSH) * C::B;
+  return pos * C::PITCH + b + (pos / tile_first<C>::value) * C::B;
+}
+template <class C> constexpr int tile_step(int pos) {  // of a multiple of R0
+  return pos * C::PITCH + (pos / tile_first<C>::value) * C::B;
 }
 
 template <class C, int R, int NS>
 __device__ __forceinline__ void tile_put(cpx<typename C::real>* lds, const cpx<typename C::real>* v, int t, int b) {
-  for_layout<C, R>(t, [&](auto slot, u32 n) {
-    constexpr int W = C::N / R;
-    constexpr int r = decltype(slot)::value % R;
-    const int j = (int)n - r * W;
-    lds[tile_addr<C>(b, (j / NS) * NS * R + (j % NS) + r * NS)] = v[decltype(slot)::value];
+  constexpr int W = C::N / R, Q = (W + C::TT - 1) / C::TT;
+  sfor<0, Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    const int j = t + q * C::TT;
+    if ((q + 1) * C::TT <= W || j < W) {
+      const int base = NS == 1 ? j * R : (j / NS) * NS * R + j % NS;
+      cpx<typename C::real>* p = lds + tile_addr<C>(b, base);
+      sfor<0, R>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        if constexpr (NS % tile_first<C>::value == 0) p[tile_step<C>(r * NS)] = v[q * R + r];
+        else if constexpr (NS == 1 && R == tile_first<C>::value) p[r * C::PITCH] = v[q * R + r];
+        else lds[tile_addr<C>(b, base + r * NS)] = v[q * R + r];
+      });
+    }
   });
 }
 
 template <class C, int R>
 __device__ __forceinline__ void tile_get(const cpx<typename C::real>* lds, cpx<typename C::real>* v, int t, int b) {
-  for_layout<C, R>(t, [&](auto slot, u32 n) { v[decltype(slot)::value] = lds[tile_addr<C>(b, (int)n)]; });
+  constexpr int W = C::N / R, Q = (W + C::TT - 1) / C::TT;
+  sfor<0, Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    const int j = t + q * C::TT;
+    if ((q + 1) * C::TT <= W || j < W) {
+      const cpx<typename C::real>* p = lds + tile_addr<C>(b, j);
+      sfor<0, R>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        if constexpr (W % tile_first<C>::value == 0) v[q * R + r] = p[tile_step<C>(r * W)];
+        else v[q * R + r] = lds[tile_addr<C>(b, j + r * W)];
+      });
+    }
+  });
 }
 
 // The pass list on a tile.  (t, b): position of the thread while neighbours hold
-// neighbouring transforms; (tl, bl): its position in the last pass.
+// neighbouring transforms; (tl, bl): its position in the last pass.  A thread that is not
+// `on` only meets the barriers.
 template <class C, int DIR, class Cur, class... Rest>
 __device__ __forceinline__ void tile_passes_(cpx<typename C::real>* v, cpx<typename C::real>* lds, int t, int b,
-                                             int tl, int bl, const cpx<typename C::real>* tw) {
-  pass_compute<C, Cur::R, Cur::NS, DIR>(v, t, tw);
+                                             int tl, int bl, const cpx<typename C::real>* tw, bool on) {
+  if (on) pass_compute<C, Cur::R, Cur::NS, DIR>(v, t, tw);
   if constexpr (sizeof...(Rest) > 0) {
     using Nx = typename pl_first<PL<Rest...>>::type;
     constexpr bool last = sizeof...(Rest) == 1;
-    tile_put<C, Cur::R, Cur::NS>(lds, v, t, b);
+    if (on) tile_put<C, Cur::R, Cur::NS>(lds, v, t, b);
     __syncthreads();
     const int tn = last ? tl : t, bn = last ? bl : b;
-    tile_get<C, Nx::R>(lds, v, tn, bn);
+    if (on) tile_get<C, Nx::R>(lds, v, tn, bn);
     if constexpr (!last) __syncthreads();
-    tile_passes_<C, DIR, Rest...>(v, lds, tn, bn, tl, bl, tw);
+    tile_passes_<C, DIR, Rest...>(v, lds, tn, bn, tl, bl, tw, on);
   }
 }
 template <class C, int DIR, class... Ps>
 __device__ __forceinline__ void tile_passes(PL<Ps...>, cpx<typename C::real>* v, cpx<typename C::real>* lds, int t,
-                                            int b, int tl, int bl, const cpx<typename C::real>* tw) {
-  tile_passes_<C, DIR, Ps...>(v, lds, t, b, tl, bl, tw);
+                                            int b, int tl, int bl, const cpx<typename C::real>* tw, bool on = true) {
+  tile_passes_<C, DIR, Ps...>(v, lds, t, b, tl, bl, tw, on);
 }
 
 // Columns.  C: N = n1, N2, B (columns of a tile), B2 (rows of a tile of the second

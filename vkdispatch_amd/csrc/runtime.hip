@@ -108,14 +108,38 @@ __global__ void outer_roots_kernel(T* out, int rows, int cols, int step, int n) 
   out[2 * i + 1] = (T)s;
 }
 
-// dst[i] = sum_b src[b * count + i] (fixed summation order: deterministic)
-template <typename T>
+// dst[i] = sum_b src[b * count + i] (fixed summation order: deterministic), V values (16
+// bytes where count and the pointers allow) per thread, eight loads in flight.
+template <typename T, int V>
 __global__ void batch_sum_kernel(T* __restrict__ dst, const T* __restrict__ src, int batch, long long count) {
+  struct alignas(sizeof(T) * V) Vec { T v[V]; };
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  T acc = src[i];
-  for (int b = 1; b < batch; ++b) acc += src[(long long)b * count + i];
-  dst[i] = acc;
+  if (i * V >= count) return;
+  const Vec* s = reinterpret_cast<const Vec*>(src) + i;
+  const long long step = count / V;
+  Vec acc = *s;
+#pragma unroll 8
+  for (int b = 1; b < batch; ++b) {
+    const Vec x = s[(long long)b * step];
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc.v[j] += x.v[j];
+  }
+  reinterpret_cast<Vec*>(dst)[i] = acc;
+}
+
+template <typename T>
+void batch_sum_launch(uint64_t dst, uint64_t src, int batch, long long count, hipStream_t s) {
+  constexpr int V = 16 / sizeof(T);
+  const int threads = 256;
+  const bool wide = count % V == 0 && dst % 16 == 0 && src % 16 == 0;
+  const long long items = wide ? count / V : count;
+  const dim3 grid((unsigned)((items + threads - 1) / threads));
+  if (wide)
+    hipLaunchKernelGGL((batch_sum_kernel<T, V>), grid, dim3(threads), 0, s, reinterpret_cast<T*>(dst),
+                       reinterpret_cast<const T*>(src), batch, count);
+  else
+    hipLaunchKernelGGL((batch_sum_kernel<T, 1>), grid, dim3(threads), 0, s, reinterpret_cast<T*>(dst),
+                       reinterpret_cast<const T*>(src), batch, count);
 }
 
 // w[m] = exp(sign * i * pi * m^2 / n) with m^2 reduced mod 2n in integers.
@@ -491,14 +515,8 @@ int vkx_outer_roots(uint64_t dst, int rows, int cols, int step, int n, int doubl
 int vkx_batch_sum(uint64_t dst, uint64_t src, int batch, long long count, int double_precision, uint64_t stream) {
   if (batch < 1 || count < 0) return fail("vkx_batch_sum", "bad size");
   if (count == 0) return 0;
-  const int threads = 256;
-  const long long blocks = (count + threads - 1) / threads;
-  if (double_precision)
-    hipLaunchKernelGGL(batch_sum_kernel<double>, dim3((unsigned)blocks), dim3(threads), 0, S(stream),
-                       reinterpret_cast<double*>(dst), reinterpret_cast<const double*>(src), batch, count);
-  else
-    hipLaunchKernelGGL(batch_sum_kernel<float>, dim3((unsigned)blocks), dim3(threads), 0, S(stream),
-                       reinterpret_cast<float*>(dst), reinterpret_cast<const float*>(src), batch, count);
+  if (double_precision) batch_sum_launch<double>(dst, src, batch, count, S(stream));
+  else batch_sum_launch<float>(dst, src, batch, count, S(stream));
   VKX_HIP(hipGetLastError());
   return 0;
 }

@@ -48,9 +48,9 @@ def _groupings(factors: Tuple[int, ...], count: int) -> Iterator[Tuple[int, ...]
 
 
 @lru_cache(maxsize=None)
-def tile_radices(n: int) -> Optional[Tuple[Tuple[int, ...], int, float]]:
+def tile_radices(n: int, most: int = MAX_RADIX) -> Optional[Tuple[Tuple[int, ...], int, float]]:
     """(radices, threads per transform, waste) of an n-point transform in registers: the
-    fewest passes, then the least idle work.  ``waste`` is the butterflies' slots over
+    fewest passes with at most ``most`` values per thread, then the least idle work.  ``waste`` is the butterflies' slots over
     their values (1: every thread has a full set in every pass)."""
     for count in (2, 3, 4):
         best = None
@@ -59,7 +59,7 @@ def tile_radices(n: int) -> Optional[Tuple[Tuple[int, ...], int, float]]:
             if count > 2 and max(rads) > 16 and n <= 16 ** count:
                 continue
             for tt in sorted({n // (r * q) for r in rads for q in (1, 2, 3, 4) if n // (r * q) >= 4}):
-                if tt > MAX_THREADS // 4 or max(slots(n, r, tt) for r in rads) > MAX_RADIX:
+                if tt > MAX_THREADS // 4 or max(slots(n, r, tt) for r in rads) > most:
                     continue
                 waste = sum(slots(n, r, tt) * tt for r in rads) / (n * count)
                 key = (round(waste, 2), max(rads), -tt)
@@ -84,12 +84,8 @@ class TilePlan:
         return self.B + 1 if self.turned else self.B
 
     @property
-    def lsh(self) -> int:
-        return int(math.log2(self.radices[0]))
-
-    @property
     def lds_elems(self) -> int:
-        return (self.N - 1) * self.pitch + ((self.N - 1) >> self.lsh) * self.B + self.B
+        return (self.N - 1) * self.pitch + (self.N - 1) // self.radices[0] * self.B + self.B
 
     @property
     def lds_bytes(self) -> int:
@@ -157,7 +153,7 @@ def _cfg(tile: TilePlan, n1: int, n2: int, b2: int, ys: int, nwg: int, tiles: in
         "  using real = float;",
         f"  static constexpr int N = {tile.N}, TT = {tile.TT}, B = {tile.B}, BLOCK = {tile.TT * tile.B}, "
         f"VMAX = {tile.vmax};",
-        f"  static constexpr int PITCH = {tile.pitch}, LSH = {tile.lsh}, LDS_ELEMS = {tile.lds_elems};",
+        f"  static constexpr int PITCH = {tile.pitch}, LDS_ELEMS = {tile.lds_elems};",
         f"  static constexpr int N1 = {n1}, N2 = {n2}, B2 = {b2}, TILES = {tiles};",
         f"  static constexpr vkx::u64 YS = {ys}ull;",
         f"  static constexpr bool INV = {flag(inverse)}, NORMALIZE = {flag(normalize)};",

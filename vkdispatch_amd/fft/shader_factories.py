@@ -118,12 +118,13 @@ def make_fft_shader(buffer_shape: Tuple, axis: int = None, inverse: bool = False
 
 def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: bool, io_type, compute_type,
                           input_signal_range, oop: bool = False, real_pitch: Optional[int] = None,
-                          spec_pitch: Optional[int] = None) -> CompiledKernel:
+                          spec_pitch: Optional[int] = None, packed: bool = False) -> CompiledKernel:
     """r2c / c2r of even-length rows through an N/2-point complex FFT (rfft_body / irfft_body).
 
     In place on an RFFTBuffer by default.  ``oop``: the real rows live in a separate
     buffer of row pitch ``real_pitch`` reals (slot 1 for r2c input, slot 0 for c2r
-    output) and the spectrum in one of row pitch ``spec_pitch`` complex values."""
+    output) and the spectrum in one of row pitch ``spec_pitch`` complex values.
+    ``packed``: a row's spectrum is N/2 values, X_0 + i X_(N/2) in the first."""
     N = geom.N
     M = N // 2
     half_geom = AxisGeometry((geom.OUTER, M), 1, M, 1, geom.OUTER)
@@ -138,6 +139,8 @@ def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: 
     # spectra measured slower (67.1 / 57.2 against 61.6 / 54.2 us)
     cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=0, sig=sig, r2c=True, inverse=inverse,
                      normalize=normalize, scale=1.0 / N)
+    if packed:
+        cfg = cfg.replace("struct Cfg {", "struct Cfg {\n  static constexpr bool PACKED = true;", 1)
     from .hooks import Arg
     if oop:
         real_t = io_type.child_type
@@ -147,7 +150,7 @@ def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: 
         args = [Arg("output", "buffer", io_type, 0)]
     kind = "irfft" if inverse else "rfft"
     body = f"vkx::{kind}_body<Cfg, {io_type.child_type.cpp}, {'true' if oop else 'false'}>(prm);"
-    tag = ("inv" if inverse else "fwd") + ("_oop" if oop else "")
+    tag = ("inv" if inverse else "fwd") + ("_oop" if oop else "") + ("_packed" if packed else "")
     src = translation_unit(cfg, [], body, plan.BLOCK, kernel_symbol(kind + "h", plan, tag))
     return CompiledKernel(src, plan, args, list(plan.radices), None, name=f"{kind}_shader_{geom.shape}",
                           roots_n=N)
@@ -156,13 +159,13 @@ def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: 
 @lru_cache(maxsize=None)
 def make_real_rows_shader(real_shape: Tuple, inverse: bool, normalize: bool = True, io_type=dt.complex64,
                           compute_type=dt.complex64, oop: bool = False, real_pitch: Optional[int] = None,
-                          spec_pitch: Optional[int] = None) -> CompiledKernel:
+                          spec_pitch: Optional[int] = None, packed: bool = False) -> CompiledKernel:
     """Row r2c / c2r kernel for even row length (internal building block of fused paths)."""
     geom = AxisGeometry.of(tuple(real_shape), None)
     if geom.N % 2:
         raise ValueError("real-row kernels need an even row length")
     return _make_real_row_shader(geom, inverse, normalize, io_type, compute_type, None, oop, real_pitch,
-                                 spec_pitch)
+                                 spec_pitch, packed)
 
 
 @lru_cache(maxsize=None)
