@@ -176,3 +176,34 @@ def test_timed_launches_match_plain_launches():
     ms = [a.elapsed_ms(b) for a, b in evs]
     print(f"  kernel ms {ms}", flush=True)
     assert all(0.0 < t < 100.0 for t in ms)
+
+
+@pytest.mark.parametrize("shape", [(256, 128, 128), (3, 64, 64), (5, 2, 4), (2, 13, 6), (7, 60, 100), (100, 210, 98),
+                                   (1, 32, 256), (2, 256, 32), (97, 96, 120), (3, 16, 210)])
+@pytest.mark.parametrize("per_image", [False, True])
+def test_one_workgroup_per_image(shape, per_image):
+    """Odd numbers of columns (M = 3, 49, 105), one-pass rows or columns, lines that do not
+    fill a wave, two images to a CU, a kernel per image; kernel spectra that are no real
+    kernel's (columns 0 and W/2 not Hermitian), unnormalised too; replayed in a graph."""
+    rng = np.random.default_rng(shape[1] * 1000 + shape[2])
+    b, h, w = shape
+    x = rng.uniform(-1, 1, shape).astype(np.float32)
+    kshape = (b if per_image else 1, h, w // 2 + 1)
+    K = (rng.standard_normal(kshape) + 1j * rng.standard_normal(kshape)).astype(np.complex64)
+    kb = vd.RFFTBuffer((kshape[0], h, w) if per_image else (h, w))
+    kb.write_fourier(K if per_image else K[0])
+    buf = vd.asrfftbuffer(x)
+    plan = fused.fused_eligible(buf, kb, kernel_inner_only=not per_image)
+    assert type(plan).__name__ == "HalfWhole"
+    ref = np.fft.irfft2(np.fft.rfft2(x.astype(np.float64)) * np.conj(K.astype(np.complex128)), s=(h, w))
+    vd.fft.convolve2DR(buf, kb, kernel_inner_only=not per_image)
+    assert O.rel_l2(buf.read_real(0), ref) < 1e-6
+    buf.write_real(x)
+    vd.fft.convolve2DR(buf, kb, kernel_inner_only=not per_image, normalize=False)
+    assert O.rel_l2(buf.read_real(0), ref * (h * w)) < 1e-6
+    g = vd.CommandGraph()
+    vd.fft.convolve2DR(buf, kb, kernel_inner_only=not per_image, graph=g)
+    for _ in range(3):
+        buf.write_real(x)
+        g.submit()
+        assert O.rel_l2(buf.read_real(0), ref) < 1e-6

@@ -135,8 +135,7 @@ __device__ __forceinline__ void pair_add_product(cpx<T>* sum, const cpx<T>* x, c
 
 // Convolution down the columns: FFT . K . IFFT, in place.  C: N = H, M, SP, B, TILES,
 // IMAGES, PER (images per workgroup, one after another with K in registers), GROUPS =
-// ceil(IMAGES / PER), KHALF, CONJ, KSTEP (elements from one image's K to the next; 0:
-// one for all), SCALE, KEEP (the transforms are also stored).  Slots: 0 spectra, 1 K, 2 the
+// ceil(IMAGES / PER), KHALF, CONJ, SCALE, KEEP (the transforms are also stored).  Slots: 0 spectra, 1 K, 2 the
 // transforms.
 template <class C, class T>
 __device__ __forceinline__ void half_conv_body(const KParams& prm) {
@@ -151,11 +150,8 @@ __device__ __forceinline__ void half_conv_body(const KParams& prm) {
   const cpx<T>* twf = bufp<const cpx<T>>(prm, SLOT_TW_FWD);
   const cpx<T>* twi = bufp<const cpx<T>>(prm, SLOT_TW_INV);
   cpx<T> kv[C::VMAX];
-  auto load_k = [&](const HalfKernel<C, T>& k) {
-    for_layout<C, FL::R>(w.t, [&](auto slot, u32 n) { kv[decltype(slot)::value] = k.plain(n, w.col); });
-  };
-  HalfKernel<C, T> k{bufp<const cpx<T>>(prm, 1)};
-  if constexpr (C::KSTEP == 0 && C::PER > 1) load_k(k);
+  const HalfKernel<C, T> k{bufp<const cpx<T>>(prm, 1)};
+  for_layout<C, FL::R>(w.t, [&](auto slot, u32 n) { kv[decltype(slot)::value] = k.plain(n, w.col); });
 #pragma nounroll
   for (int i = 0; i < C::PER; ++i) {
     const int image = w.group * C::PER + i;
@@ -164,8 +160,6 @@ __device__ __forceinline__ void half_conv_body(const KParams& prm) {
     cpx<T>* s = bufp<cpx<T>>(prm, 0) + half_at<C>(image);
     cpx<T> v[C::VMAX];
     half_load<C, F0::R>(w, s, v);
-    if constexpr (C::KSTEP != 0) k.k = bufp<const cpx<T>>(prm, 1) + (u64)image * (u64)C::KSTEP;
-    if constexpr (C::KSTEP != 0 || C::PER == 1) load_k(k);
     tile_passes<C, -1>(L{}, v, lds, w.t, w.b, w.t, w.b, twf);
     if constexpr (C::KEEP) half_store<C, FL::R>(w, bufp<cpx<T>>(prm, 2) + half_at<C>(image), v, (T)1);
     if (w.tile == 0) {
@@ -307,6 +301,238 @@ __device__ __forceinline__ void half_grad_body(const KParams& prm) {
     for_layout<C, IL::R>(w.t, [&](auto slot, u32 n) {
       p[n * (u32)C::M + w.col] = sum[decltype(slot)::value] * (T)C::SCALE;
     });
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The whole convolution of one image in one workgroup: rows, columns . K, columns and
+// rows back, with the image in LDS in between, where three launches crossed memory three
+// times.  A line (row or column) belongs to one wave: its TT threads exchange through its
+// own LDS without a barrier, and the workgroup meets only twice, between rows and columns.
+// C: N = H, M, BLOCK, RP (pitch; chosen so that neither direction meets the same banks),
+// IMG (reals per image), RowCfg / ColCfg (N, TT, VMAX, fwd, inv), KHALF / CONJ / KSTEP
+// (elements from one image's K to the next; 0: one for all), SCALE (of the whole), ROOTS (a
+// multiple of 2M and H).  Slots: 0 images (rows of 2M + 2 reals, in place), 1 K.
+//
+// Bound by the vector unit: at 256 images of 128^2, one per CU, 19 us, of which the
+// transforms' adds and products are 8 (no packed FP32) and memory 4; three launches took 37.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <class C, int STRIDE, int R, int NS, class T>
+__device__ __forceinline__ void line_put(cpx<T>* line, const cpx<T>* v, int t) {
+  constexpr int W = C::N / R, Q = (W + C::TT - 1) / C::TT;
+  sfor<0, Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    const int j = t + q * C::TT;
+    if ((q + 1) * C::TT <= W || j < W) {
+      cpx<T>* p = line + (NS == 1 ? j * R : (j / NS) * NS * R + j % NS) * STRIDE;
+      sfor<0, R>([&](auto rc) { p[decltype(rc)::value * NS * STRIDE] = v[q * R + decltype(rc)::value]; });
+    }
+  });
+}
+template <class C, int STRIDE, int R, class T>
+__device__ __forceinline__ void line_get(const cpx<T>* line, cpx<T>* v, int t) {
+  constexpr int W = C::N / R, Q = (W + C::TT - 1) / C::TT;
+  sfor<0, Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    const int j = t + q * C::TT;
+    if ((q + 1) * C::TT <= W || j < W) {
+      const cpx<T>* p = line + j * STRIDE;
+      sfor<0, R>([&](auto rc) { v[q * R + decltype(rc)::value] = p[decltype(rc)::value * W * STRIDE]; });
+    }
+  });
+}
+// f(slot, row, column) over `have` rows of M values, lane by lane: one division per call,
+// then steps.
+template <int M, int IT, class F> __device__ __forceinline__ void row_points(int lane, int have, F&& f) {
+  int y = lane / M, n = lane % M;
+  sfor<0, IT>([&](auto ic_) {
+    if (y < have) f(ic_, y, n);
+    n += 64 % M;
+    y += 64 / M;
+    if (64 % M != 0 && n >= M) { n -= M; y += 1; }
+  });
+}
+
+// The twiddle table of a pass list (see pass_compute) from the roots of order C::ROOTS.
+template <class L> struct list_twiddles;
+template <class... Ps> struct list_twiddles<PL<Ps...>> { static constexpr int value = (0 + ... + ((Ps::R - 1) * Ps::NS)); };
+template <class C, class T, class... Ps>
+__device__ __forceinline__ void fill_twiddles(PL<Ps...>, cpx<T>* tab, const cpx<T>* roots) {
+  auto one = [&](auto rc, auto ns) {
+    constexpr int R = decltype(rc)::value, NS = decltype(ns)::value, STEP = C::ROOTS / (R * NS);
+    if constexpr (NS > 1)
+      for (int i = (int)threadIdx.x; i < (R - 1) * NS; i += C::BLOCK)
+        tab[NS - 1 + i] = roots[(i / NS + 1) * (i % NS) % (R * NS) * STEP];
+  };
+  (one(ic<Ps::R>{}, ic<Ps::NS>{}), ...);
+}
+
+// The pass list on a line, from registers (first pass's order) to registers (last pass's).
+template <class C, int STRIDE, int DIR, class T, class Cur, class... Rest>
+__device__ __forceinline__ void line_passes(PL<Cur, Rest...>, cpx<T>* v, cpx<T>* line, int t, const cpx<T>* tw, bool on) {
+  if (on) pass_compute<C, Cur::R, Cur::NS, DIR>(v, t, tw);
+  if constexpr (sizeof...(Rest) > 0) {
+    wave_sync();
+    if (on) line_put<C, STRIDE, Cur::R, Cur::NS>(line, v, t);
+    wave_sync();
+    if (on) line_get<C, STRIDE, pl_first<PL<Rest...>>::type::R>(line, v, t);
+    line_passes<C, STRIDE, DIR>(PL<Rest...>{}, v, line, t, tw, on);
+  }
+}
+
+template <class C, class T>
+__device__ __forceinline__ void half_whole_body(const KParams& prm) {
+  using RC = typename C::RowCfg;
+  using CC = typename C::ColCfg;
+  using RF = typename RC::fwd;
+  using CF = typename CC::fwd;
+  using CI = typename CC::inv;
+  __shared__ cpx<T> lds[C::N * C::RP];
+  // Twiddles and roots in LDS: a pass then waits for LDS and not for L2, and each of the
+  // passes is a link of one chain.  All come from one table of roots of order ROOTS.
+  constexpr int NR = list_twiddles<typename RC::fwd>::value, NC = list_twiddles<typename CC::fwd>::value;
+  constexpr int PAIRS = C::M / 2 + 1;
+  __shared__ cpx<T> tab[NR + 2 * NC + PAIRS];
+  const cpx<T>*row_tw = tab, *col_fwd = tab + NR, *col_inv = col_fwd + NC, *roots = col_inv + NC;
+  {
+    const cpx<T>* w = bufp<const cpx<T>>(prm, SLOT_ROOTS);
+    fill_twiddles<C>(RF{}, tab, w);
+    fill_twiddles<C>(CF{}, tab + NR, w);
+    fill_twiddles<C>(CI{}, tab + NR + NC, w);
+    for (int i = (int)threadIdx.x; i < PAIRS; i += C::BLOCK) tab[NR + 2 * NC + i] = w[i * (C::ROOTS / (2 * C::M))];
+  }
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  constexpr int WAVES = C::BLOCK / 64;
+  constexpr int RL = 64 / RC::TT, CL = 64 / CC::TT;  // lines of a wave
+  const u32 image = blockIdx.x;
+  cpx<T>* x = reinterpret_cast<cpx<T>*>(bufp<T>(prm, 0) + (u64)image * (u64)C::IMG);
+  const HalfKernel<C, T> k{bufp<const cpx<T>>(prm, 1) + (u64)image * (u64)C::KSTEP};
+  constexpr int IT = (RL * C::M + 63) / 64;
+  int rt = lane % RC::TT, ct = lane % CC::TT;
+  __syncthreads();  // the tables
+  // addresses are computed again in each round of a loop, not held through it
+  auto forget = [&] { asm volatile("" : "+v"(rt), "+v"(ct)); };
+
+#pragma nounroll
+  for (int y0 = wave * RL; y0 < C::N; y0 += WAVES * RL) {
+    forget();
+    cpx<T>* rows = lds + y0 * C::RP;
+    const int have = (C::N - y0 < RL ? C::N - y0 : RL);
+    {
+      cpx<T> v[IT];  // the wave's rows, every load in flight before the first is waited for
+      cpx<T>* xr = x + y0 * (C::M + 1);
+      row_points<C::M, IT>(lane, have, [&](auto ic_, int y, int n) { v[decltype(ic_)::value] = xr[y * (C::M + 1) + n]; });
+      row_points<C::M, IT>(lane, have, [&](auto ic_, int y, int n) { rows[y * C::RP + n] = v[decltype(ic_)::value]; });
+    }
+    const bool on = lane < have * RC::TT;
+    cpx<T>* row = rows + lane / RC::TT * C::RP;
+    cpx<T> v[RC::VMAX];
+    wave_sync();
+    if (on) line_get<RC, 1, pl_first<RF>::type::R>(row, v, rt);
+    line_passes<RC, 1, -1, T>(RF{}, v, row, rt, row_tw, on);
+    wave_sync();
+    if (on) for_layout<RC, pl_last<RF>::type::R>(rt, [&](auto slot, u32 n) { row[n] = v[decltype(slot)::value]; });
+    wave_sync();
+    // half-length transform -> packed spectrum, q and M - q by one thread of the row
+    if (on) {
+      for (int q = rt; q < PAIRS; q += RC::TT) {
+        const cpx<T> zk = row[q], zm = row[q == 0 ? 0 : C::M - q];
+        if (q == 0) {
+          row[0] = cpx<T>{zk.x + zk.y, zk.x - zk.y};
+        } else {
+          const T h = (T)0.5;
+          const cpx<T> e{h * (zk.x + zm.x), h * (zk.y - zm.y)}, o{h * (zk.y + zm.y), h * (zm.x - zk.x)};
+          const cpx<T> w = cmul(roots[q], o);
+          row[q] = e + w;
+          if (2 * q != C::M) row[C::M - q] = conj(e - w);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+#pragma nounroll
+  for (int c0 = wave * CL; c0 < C::M; c0 += WAVES * CL) {
+    forget();
+    const int have = (C::M - c0 < CL ? C::M - c0 : CL);
+    const bool on = lane < have * CC::TT;
+    const int c = on ? c0 + lane / CC::TT : c0;
+    cpx<T>* col = lds + c;
+    cpx<T> v[CC::VMAX], kv[CC::VMAX];
+    const cpx<T>* kc = k.k + (u32)ct * HalfKernel<C, T>::KP + (u32)c;  // the legs are constants apart
+    for_layout<CC, pl_last<CF>::type::R>(0, [&](auto slot, u32 n) {
+      if (CC::N / pl_last<CF>::type::R % CC::TT == 0 || n + (u32)ct < (u32)CC::N) {
+        const cpx<T> z = kc[n * HalfKernel<C, T>::KP];
+        kv[decltype(slot)::value] = C::CONJ ? conj(z) : z;
+      }
+    });
+    if (on) line_get<CC, C::RP, pl_first<CF>::type::R>(col, v, ct);
+    line_passes<CC, C::RP, -1, T>(CF{}, v, col, ct, col_fwd, on);
+    if (c0 == 0) {  // column 0: both of its spectra, with the mirrored values from LDS
+      wave_sync();
+      if (on && c == 0)
+        for_layout<CC, pl_last<CF>::type::R>(ct, [&](auto slot, u32 n) { col[n * C::RP] = v[decltype(slot)::value]; });
+      wave_sync();
+#pragma nounroll
+      for (int n = lane; n <= C::N / 2; n += 64) {
+        const int m = n == 0 ? 0 : C::N - n;
+        cpx<T> a, b, ka, kb;
+        unpack_pair(lds[n * C::RP], lds[m * C::RP], a, b);
+        k.both((u32)n, ka, kb);
+        a = cmul(a, ka);
+        b = cmul(b, kb);
+        lds[m * C::RP] = pack_pair(conj(a), conj(b));
+        lds[n * C::RP] = pack_pair(a, b);
+      }
+      wave_sync();
+    }
+    for_layout<CC, pl_last<CF>::type::R>(ct, [&](auto slot, u32) {
+      v[decltype(slot)::value] = cmul(v[decltype(slot)::value], kv[decltype(slot)::value]);
+    });
+    if (c0 == 0 && on && c == 0)
+      for_layout<CC, pl_last<CF>::type::R>(ct, [&](auto slot, u32 n) { v[decltype(slot)::value] = col[n * C::RP]; });
+    forget();
+    line_passes<CC, C::RP, 1, T>(CI{}, v, col, ct, col_inv, on);
+    wave_sync();
+    if (on) for_layout<CC, pl_last<CI>::type::R>(ct, [&](auto slot, u32 n) { col[n * C::RP] = v[decltype(slot)::value]; });
+  }
+  __syncthreads();
+
+#pragma nounroll
+  for (int y0 = wave * RL; y0 < C::N; y0 += WAVES * RL) {
+    forget();
+    cpx<T>* rows = lds + y0 * C::RP;
+    const int have = (C::N - y0 < RL ? C::N - y0 : RL);
+    const bool on = lane < have * RC::TT;
+    cpx<T>* row = rows + lane / RC::TT * C::RP;
+    cpx<T> v[RC::VMAX];
+    if (on) {
+      for (int q = rt; q < PAIRS; q += RC::TT) {
+        const cpx<T> a = row[q], am = row[q == 0 ? 0 : C::M - q];
+        if (q == 0) {
+          row[0] = cpx<T>{a.x + a.y, a.x - a.y};
+        } else {
+          const cpx<T> e{a.x + am.x, a.y - am.y}, d{a.x - am.x, a.y + am.y};
+          const cpx<T> o = cmul(d, conj(roots[q]));
+          row[q] = e + mul_i(o);
+          if (2 * q != C::M) row[C::M - q] = conj(e + mul_negi(o));
+        }
+      }
+    }
+    wave_sync();
+    if (on) line_get<RC, 1, pl_first<RF>::type::R>(row, v, rt);
+    line_passes<RC, 1, 1, T>(RF{}, v, row, rt, row_tw, on);
+    wave_sync();
+    if (on)
+      for_layout<RC, pl_last<RF>::type::R>(rt, [&](auto slot, u32 n) { row[n] = v[decltype(slot)::value] * (T)C::SCALE; });
+    wave_sync();
+    cpx<T>* xr = x + y0 * (C::M + 1);
+    row_points<C::M, IT>(lane, have, [&](auto, int y, int n) { xr[y * (C::M + 1) + n] = rows[y * C::RP + n]; });
   }
 }
 

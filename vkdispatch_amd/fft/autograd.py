@@ -137,9 +137,9 @@ class _HalfPlans:
         self.rows_inv = make_real_rows_shader((B, H, W), True, True, c, c, True, W, M, True)
         self.rows_fwd1 = make_real_rows_shader((1, H, W), False, True, c, c, True, W, M, True)
         self.col_fft1 = make_fft_shader((1, H, M), 1, input_type=c, output_type=c, compute_type=c)
-        self.conv = half2d.make_half_conv(B, H, M, M, c, False)
-        self.conv_keep = half2d.make_half_conv(B, H, M, M, c, False, keep=True)
-        self.conv_dx = half2d.make_half_conv(B, H, M, M, c, False, False)
+        self.conv = half2d.make_half_conv(B, H, M, c)
+        self.conv_keep = half2d.make_half_conv(B, H, M, c, keep=True)
+        self.conv_dx = half2d.make_half_conv(B, H, M, c, conj=False)
         self.grad = half2d.make_half_grad(B, H, M, c)
         self.rows_inv1 = make_real_rows_shader((1, H, W), True, True, c, c, True, W, M, True)
 

@@ -1,15 +1,15 @@
 """2-D real FFT-convolution (convolve2DR) execution paths and their profiling.
 
-``try_convolve2DR`` runs the pair-packed kernels (``csrc/device/vkx_conv2d.h``)
-when the call is eligible: a batch of square real images (256, 512 or 1024 on a
-side) in complex64 RFFTBuffers, one kernel spectrum broadcast over the batch,
-the default kernel map.  It returns False otherwise, and the caller falls back
-to the reference's three-dispatch composition (rfft -> convolve(axis ndim-2) ->
-irfft, vkdispatch/fft/functions.py:614-646).  Both paths compute
-irfft2(rfft2(x) . conj(K)) per image (vkdispatch/fft/shader_factories.py:136-145).
-
-The pair-packed form is ``Conv2DPhases``: three kernels in stream order through a
-scratch image per pair.  VKX_FUSED_CONV=0 forces the three-dispatch composition.
+``try_convolve2DR`` runs complex64 RFFTBuffers with the default kernel map
+* as one workgroup per image (``half2d.HalfWhole``, csrc/device/vkx_half.h) where the
+  image fits LDS and there are enough of them (``half2d.whole_pays``);
+* as the pair-packed kernels (``Conv2DPhases``, csrc/device/vkx_conv2d.h: three kernels in
+  stream order through a scratch image per pair) for square images of 256, 512 or 1024
+  and one kernel spectrum.
+It returns False otherwise, and the caller falls back to the reference's three-dispatch
+composition (rfft -> convolve(axis ndim-2) -> irfft, vkdispatch/fft/functions.py:614-646).
+All compute irfft2(rfft2(x) . conj(K)) per image (vkdispatch/fft/shader_factories.py:136-145).
+VKX_FUSED_CONV=0 forces the three-dispatch composition.
 """
 from __future__ import annotations
 
@@ -22,8 +22,9 @@ from .. import dtypes as dt
 from .. import runtime as rt
 from ..buffer import Buffer
 from ..graph import dispatch
+from . import half2d
 from .hooks import Arg
-from .kernels import CompiledKernel, check_no_spill, kernel_symbol, source_symbol
+from .kernels import CompiledKernel, SpillError, check_no_spill, kernel_symbol, source_symbol
 from .planner import KernelPlan
 from .shader_factories import make_convolution_shader, make_fft_shader, register_plan_cache
 
@@ -183,11 +184,27 @@ def fused_plan(batch: int, H: int, W: int, normalize: bool = True):
 register_plan_cache(fused_plan.cache_clear)
 
 
+@lru_cache(maxsize=32)
+def whole_plan(batch: int, H: int, W: int, per_image: bool, normalize: bool):
+    """The one-launch plan of small images, or None where it does not fit or not pay."""
+    if W % 2 or not half2d.whole_pays(batch, H, W // 2):
+        return None
+    plan = half2d.HalfWhole(batch, H, W // 2, H * (W // 2 + 1) if per_image else 0, normalize)
+    try:
+        check_no_spill(plan.kernel)
+    except SpillError:
+        return None
+    return plan
+
+
+register_plan_cache(whole_plan.cache_clear)
+
+
 def plan_for_shape(real_shape, kernel_map=None, transposed_kernel=False, kernel_inner_only=False, normalize=True,
                    compute_type=None):
-    """The pair-packed plan for a convolve2DR over complex64 RFFTBuffers of ``real_shape``
-    with a kernel spectrum of one image, or None when the call takes the reference's
-    three-dispatch composition."""
+    """The plan for a convolve2DR over complex64 RFFTBuffers of ``real_shape`` (one workgroup
+    per small image, or the pair-packed kernels with a kernel spectrum of one image), or
+    None when the call takes the reference's three-dispatch composition."""
     if not _fused_enabled() or kernel_map is not None or transposed_kernel:
         return None
     if compute_type is not None and compute_type is not dt.complex64:
@@ -197,17 +214,17 @@ def plan_for_shape(real_shape, kernel_map=None, transposed_kernel=False, kernel_
         return None
     H, W = rs[-2], rs[-1]
     batch = rs[0] if len(rs) == 3 else 1
+    # without kernel_inner_only the reference reads one kernel spectrum per image
+    per_image = batch > 1 and not kernel_inner_only
     if H != W or W not in _FUSED_RADICES:
-        return None
-    if batch > 1 and not kernel_inner_only:
-        return None  # the reference then reads one kernel spectrum per image
-    return fused_plan(batch, H, W, bool(normalize))
+        return whole_plan(batch, H, W, per_image, bool(normalize))
+    return None if per_image else fused_plan(batch, H, W, bool(normalize))
 
 
 def fused_eligible(buffer, kernel, kernel_map=None, buffer_shape=None, transposed_kernel=False,
                    kernel_inner_only=False, normalize=True, compute_type=None, **_):
-    """The pair-packed plan (Conv2DPhases) for this convolve2DR call, or None when the
-    call needs the three-dispatch composition."""
+    """The plan (Conv2DPhases, or half2d.HalfWhole) for this convolve2DR call, or None when
+    the call needs the three-dispatch composition."""
     if getattr(buffer, "var_type", None) is not dt.complex64 or getattr(kernel, "var_type", None) is not dt.complex64:
         return None
     rs = tuple(getattr(buffer, "real_shape", ()))
@@ -215,7 +232,8 @@ def fused_eligible(buffer, kernel, kernel_map=None, buffer_shape=None, transpose
         return None
     H, W = rs[-2], rs[-1]
     wh = W // 2 + 1
-    if kernel.size < H * wh:
+    images = rs[0] if len(rs) == 3 and not kernel_inner_only else 1  # kernel spectra read
+    if kernel.size < images * H * wh:
         return None
     if len(rs) == 3 and rs[0] > 1 and tuple(kernel.shape[-2:]) != (H, wh):
         return None
@@ -229,7 +247,9 @@ def try_convolve2DR(buffer, kernel, graph=None, print_shader=False, **kw) -> boo
     if print_shader:
         for k in plan.kernels():
             print(k.source)
-    plan(buffer, kernel, graph)
+    vals = plan.values(buffer, kernel)
+    for k in plan.kernels():
+        dispatch(k, vals, graph)
     return True
 
 

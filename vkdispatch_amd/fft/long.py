@@ -30,7 +30,7 @@ TILE_MAX = 4096       # longest column or row: 4 of them (32-byte runs) still fi
 CHUNK_POINTS = 1 << 23  # points per pair of launches: 64 MiB of scratch, which stays in the 256 MB cache
 
 
-def _groupings(factors: Tuple[int, ...], count: int) -> Iterator[Tuple[int, ...]]:
+def groupings(factors: Tuple[int, ...], count: int) -> Iterator[Tuple[int, ...]]:
     """The ways to write the product of ``factors`` as ``count`` radices of at most
     MAX_RADIX, largest first."""
     n = math.prod(factors)
@@ -54,7 +54,7 @@ def tile_radices(n: int, most: int = MAX_RADIX) -> Optional[Tuple[Tuple[int, ...
     their values (1: every thread has a full set in every pass)."""
     for count in (2, 3, 4):
         best = None
-        for rads in _groupings(tuple(prime_factors(n)), count):
+        for rads in groupings(tuple(prime_factors(n)), count):
             # three passes need no large radices, and these cost registers
             if count > 2 and max(rads) > 16 and n <= 16 ** count:
                 continue

@@ -125,8 +125,8 @@ def convolve2D_src(buffer_shape, kernel_map=None, normalize=True, transposed_ker
 def convolve2DR_src(buffer_shape, kernel_map=None, transposed_kernel=False, kernel_inner_only=False,
                     normalize=True) -> Tuple[str, ...]:
     """The kernels convolve2DR launches for complex64 RFFTBuffers of ``buffer_shape`` (the
-    real shape) with one kernel spectrum: the pair-packed kernels when the call takes
-    that path (one source for the single launch, three for the phase kernels), else the
+    real shape): one kernel for small images that take a workgroup each, the three
+    pair-packed kernels when the call takes that path (one kernel spectrum), else the
     reference's rfft -> convolve -> irfft composition."""
     _check_dims(buffer_shape, (2, 3), "Buffer")
     from . import fused
