@@ -315,16 +315,29 @@ template <class C> __device__ __forceinline__ u32 logical_wg() {
   }
 }
 
+// C::LPW (optional, WAVE_LOCAL): a wave takes LPW transforms of TT threads and its last
+// lanes have none; they leave at once (such a kernel has no barriers).
+template <class C, class = void> struct lpw_of { static constexpr int value = 0; };
+template <class C> struct lpw_of<C, decltype((void)C::LPW)> { static constexpr int value = C::LPW; };
+template <class C> __device__ __forceinline__ bool idle_lane() {
+  if constexpr (lpw_of<C>::value > 0) return (int)(threadIdx.x & 63u) >= C::LPW * C::TT;
+  else return false;
+}
+
 template <class C> __device__ __forceinline__ Geo make_geo() {
   Geo g;
   const int tid = (int)threadIdx.x;
-  if constexpr (C::COLFAST) { g.b = tid % C::B; g.t = tid / C::B; }
+  if constexpr (lpw_of<C>::value > 0) {
+    const int lane = tid & 63;
+    g.t = lane % C::TT;
+    g.b = (tid >> 6) * C::LPW + lane / C::TT;
+  } else if constexpr (C::COLFAST) { g.b = tid % C::B; g.t = tid / C::B; }
   else { g.t = tid % C::TT; g.b = tid / C::TT; }
   const u32 wg = logical_wg<C>();
   if constexpr (C::S > 1) {
     g.outer = wg / C::NWG_INNER;
     g.inner = (wg % C::NWG_INNER) * C::B + (u32)g.b;
-    g.valid = g.inner < C::S;
+    g.valid = g.inner < C::S && g.outer < C::OUTER;  // (the grid may end in idle workgroups)
   } else {
     g.outer = wg * C::B + (u32)g.b;
     g.inner = 0;
@@ -444,11 +457,30 @@ template <int SLOT, class S> struct DefaultKernel {
 
 // ---------------------------------------------------------------------------
 // LDS addressing.  COLFAST (strided axes, transform slot fastest across lanes):
-// element (b, pos) at pos*B + b.  Otherwise one padded row per transform.
+// element (b, pos) at pos*B + b; with C::CPAD (optional) moved on by B for every R0
+// positions (R0: the first radix), since in the first exchange neighbouring threads write
+// R0 positions apart and would meet the same banks.  Otherwise one padded row per transform.
 // ---------------------------------------------------------------------------
+template <class C, class = void> struct cpad_of { static constexpr int value = 0; };  // R0, 0: none
+template <class C> struct cpad_of<C, decltype((void)C::CPAD)> {
+  static constexpr int value = C::CPAD ? pl_first<typename C::fwd>::type::R : 0;
+};
 template <class C> __device__ __forceinline__ int lds_addr(int b, int pos) {
-  if constexpr (C::COLFAST) return pos * C::B + b;
+  constexpr int R0 = cpad_of<C>::value;
+  if constexpr (C::COLFAST && R0 > 0) return pos * C::B + b + pos / R0 * C::B;
+  else if constexpr (C::COLFAST) return pos * C::B + b;
   else return b * C::NP + pos + (pos >> C::PAD_SHIFT);
+}
+// Address of leg r (constant) at position base + r STEP, from leg 0's where the padding
+// makes that a constant: a step of whole periods, or the first pass's own legs.
+template <class C, int STEP, int R, bool PUT>
+__device__ __forceinline__ int lds_leg(int b, int base, int leg0, int r) {
+  constexpr int R0 = cpad_of<C>::value;
+  if constexpr (C::COLFAST && R0 > 0) {
+    if constexpr (STEP % R0 == 0) return leg0 + r * (STEP + STEP / R0) * C::B;
+    else if constexpr (PUT && STEP == 1 && R == R0) return leg0 + r * C::B;
+  }
+  return lds_addr<C>(b, base + r * STEP);
 }
 
 template <class C> __device__ __forceinline__ void block_sync() {
@@ -497,10 +529,10 @@ __device__ __forceinline__ void lds_put(cpx<typename C::real>* lds, const cpx<ty
     constexpr bool full = (q + 1) * C::TT <= W;
     const int j = t + q * C::TT;
     if (full || j < W) {
-      const int base = (j / NS) * NS * R + (j % NS);
+      const int base = (j / NS) * NS * R + (j % NS), leg0 = lds_addr<C>(b, base);
       sfor<0, R>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        lds[lds_addr<C>(b, base + r * NS)] = v[q * R + r];
+        lds[lds_leg<C, NS, R, true>(b, base, leg0, r)] = v[q * R + r];
       });
     }
   });
@@ -515,9 +547,10 @@ __device__ __forceinline__ void lds_get(const cpx<typename C::real>* lds, cpx<ty
     constexpr bool full = (q + 1) * C::TT <= W;
     const int j = t + q * C::TT;
     if (full || j < W) {
+      const int leg0 = lds_addr<C>(b, j);
       sfor<0, R>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        v[q * R + r] = lds[lds_addr<C>(b, j + r * W)];
+        v[q * R + r] = lds[lds_leg<C, W, R, false>(b, j, leg0, r)];
       });
     }
   });
@@ -681,6 +714,7 @@ __device__ __forceinline__ void fft_body(const KParams& prm) {
   using F0 = typename pl_first<L>::type;
   using FL = typename pl_last<L>::type;
   __shared__ cpx<real> lds[C::LDS_ELEMS];
+  if (idle_lane<C>()) return;
   const Geo g = make_geo<C>();
   cpx<real> v[C::VMAX];
   const cpx<real>* tw = bufp<const cpx<real>>(prm, SLOT_TW_FWD);
@@ -744,6 +778,7 @@ __device__ __forceinline__ void conv_body(const KParams& prm) {
   using FL = typename pl_last<L>::type;
   using IL = typename pl_last<LI>::type;
   __shared__ cpx<real> lds[C::LDS_ELEMS];
+  if (idle_lane<C>()) return;
   const Geo g = make_geo<C>();
   cpx<real> v[C::VMAX];
   const cpx<real>* twf = bufp<const cpx<real>>(prm, SLOT_TW_FWD);
@@ -833,6 +868,7 @@ __device__ __forceinline__ void rfft_body(const KParams& prm) {
   using FL = typename pl_last<L>::type;
   constexpr int M = C::N;
   __shared__ cpx<real> lds[C::LDS_ELEMS];
+  if (idle_lane<C>()) return;
   const Geo g = make_geo<C>();
   cpx<real> v[C::VMAX];
   const cpx<real>* tw = bufp<const cpx<real>>(prm, SLOT_TW_FWD);
@@ -893,6 +929,7 @@ __device__ __forceinline__ void irfft_body(const KParams& prm) {
   using FL = typename pl_last<L>::type;
   constexpr int M = C::N;
   __shared__ cpx<real> lds[C::LDS_ELEMS];
+  if (idle_lane<C>()) return;
   const Geo g = make_geo<C>();
   cpx<real> v[C::VMAX];
   const cpx<real>* tw = bufp<const cpx<real>>(prm, SLOT_TW_FWD);
@@ -940,6 +977,7 @@ __device__ __forceinline__ void irfft_body(const KParams& prm) {
 template <class C, class SIn, class SOut>
 __device__ __forceinline__ void transpose_body(const KParams& prm) {
   using FL = typename pl_last<typename C::fwd>::type;
+  if (idle_lane<C>()) return;
   const Geo g = make_geo<C>();
   if (!g.valid) return;
   if constexpr (C::KERNEL_INNER_ONLY) {

@@ -12,9 +12,8 @@ import numpy as np
 from .. import dtypes as dt
 from .hooks import Arg
 from .kernels import CompiledKernel, kernel_symbol, translation_unit
-from .long import TilePlan, groupings, tile_radices
-from .planner import LDS_BYTES_MAX, MAX_THREADS, KernelPlan, pass_list, slots
-from .prime_utils import prime_factors
+from .long import TilePlan, tile_radices
+from .planner import LDS_BYTES_MAX, MAX_THREADS, KernelPlan, groupings, pass_list, slots
 from .precision import kernel_real_type
 
 LDS_SHARED = 80 * 1024  # two workgroups on a CU
@@ -110,9 +109,7 @@ def _line_radices(n: int, lines: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     workgroup over all ``lines`` (16 waves of 8 values 21 us, 8 waves of 16 values 23 us)."""
     for count in (1, 2, 3, 4):
         best = None
-        for rads in groupings(tuple(prime_factors(n)), count):
-            if max(rads) > 16:
-                continue
+        for rads in groupings(n, count, 16):
             for tt in sorted({-(-n // (r * q)) for r in rads for q in (1, 2)}):
                 values = max(slots(n, r, tt) for r in rads)
                 if tt > 64 or values > 20:

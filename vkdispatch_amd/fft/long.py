@@ -14,37 +14,20 @@ import dataclasses
 import math
 import threading
 from functools import lru_cache
-from typing import Dict, Iterator, List, Optional, Tuple
+from typing import Dict, List, Optional, Tuple
 
 from .. import dtypes as dt
 from .. import runtime as rt
 from ..buffer import Buffer
 from .hooks import Arg
 from .kernels import CompiledKernel, check_no_spill, kernel_symbol, translation_unit
-from .planner import LDS_BYTES_MAX, MAX_THREADS, KernelPlan, pass_list, slots
+from .planner import LDS_BYTES_MAX, MAX_THREADS, KernelPlan, groupings, pass_list, slots
 from .prime_utils import prime_factors
 
 MAX_PRIME = 13        # larger prime factors go through Bluestein (fft/ragged.py)
 MAX_RADIX = 32        # complex64 values a thread holds at most (64 registers)
 TILE_MAX = 4096       # longest column or row: 4 of them (32-byte runs) still fit LDS
 CHUNK_POINTS = 1 << 23  # points per pair of launches: 64 MiB of scratch, which stays in the 256 MB cache
-
-
-def groupings(factors: Tuple[int, ...], count: int) -> Iterator[Tuple[int, ...]]:
-    """The ways to write the product of ``factors`` as ``count`` radices of at most
-    MAX_RADIX, largest first."""
-    n = math.prod(factors)
-
-    def rec(rest: int, k: int, most: int):
-        if k == 1:
-            if 1 < rest <= most:
-                yield (rest,)
-            return
-        for r in range(min(most, rest // 2 ** (k - 1)), 1, -1):
-            if rest % r == 0:
-                for tail in rec(rest // r, k - 1, r):
-                    yield (r,) + tail
-    yield from rec(n, count, MAX_RADIX)
 
 
 @lru_cache(maxsize=None)
@@ -54,7 +37,7 @@ def tile_radices(n: int, most: int = MAX_RADIX) -> Optional[Tuple[Tuple[int, ...
     their values (1: every thread has a full set in every pass)."""
     for count in (2, 3, 4):
         best = None
-        for rads in groupings(tuple(prime_factors(n)), count):
+        for rads in groupings(n, count, MAX_RADIX):
             # three passes need no large radices, and these cost registers
             if count > 2 and max(rads) > 16 and n <= 16 ** count:
                 continue

@@ -18,7 +18,8 @@ from __future__ import annotations
 import dataclasses
 import math
 import os
-from typing import List, Optional, Tuple
+from functools import lru_cache
+from typing import Iterator, List, Optional, Tuple
 
 from .prime_utils import prime_factors
 
@@ -39,6 +40,85 @@ _POW2 = {
 
 def _wave_local_default() -> bool:
     return os.environ.get("VKX_WAVE_LOCAL", "1") != "0"
+
+
+def groupings(n: int, count: int, most: int) -> Iterator[Tuple[int, ...]]:
+    """The ways to write n as a product of ``count`` radices of at most ``most``, largest first."""
+    def rec(rest: int, k: int, top: int):
+        if k == 1:
+            if 1 < rest <= top:
+                yield (rest,)
+            return
+        for r in range(min(top, rest // 2 ** (k - 1)), 1, -1):
+            if rest % r == 0:
+                for tail in rec(rest // r, k - 1, r):
+                    yield (r,) + tail
+    yield from rec(n, count, most)
+
+
+@lru_cache(maxsize=None)
+def balanced_plan(N: int, elem: int) -> Optional[Tuple[Tuple[int, ...], int]]:
+    """(radices, threads) of contiguous transforms whose length is no power of two: the
+    least cost of the fewest passes, the idle slots and lanes in them, registers, barriers
+    and short runs.  The weights are fitted to 1080 kernels of 61 lengths of 60 to 15000
+    points, 50 MB in and out (MI355X): the picks are 1.3 % above the best of each length, the
+    former rule (first-fit packing into radices up to 16, N / largest radix threads)
+    26 %.  600 points 12.1 -> 10.3 us, 2160 17.0 -> 10.3, 480 15.3 -> 9.1; complex128 of
+    600 points 12.7 -> 8.5, 2400 16.0 -> 10.2."""
+    dbl = elem == 16
+    most = 16 if dbl else 32     # values per thread: 64 registers
+    if dbl and max(prime_factors(N)) > most:
+        return None              # a butterfly of 17 or more complex128 needs more than that
+    best = None
+    for count in (2, 3, 4, 5):
+        for rads in groupings(N, count, max(most, MAX_DIRECT_PRIME)):
+            if any(r > most and len(prime_factors(r)) > 1 for r in rads):
+                continue
+            for order in {rads, rads[::-1]}:
+                for tt in {-(-N // (r * q)) for r in rads for q in (1, 2, 3)}:
+                    values = max(slots(N, r, tt) for r in order)
+                    # 1024 threads leave 128 registers each, 512 leave 256
+                    room = most if tt <= 512 else most // 2
+                    if tt > MAX_THREADS or values > max(room, max(rads)) or values < 4:
+                        continue
+                    lanes = WAVE / (WAVE // tt * tt) if tt <= WAVE else -(-tt // WAVE) * WAVE / tt
+                    work = sum(slots(N, r, tt) * tt for r in order) / N * lanes
+                    cost = (0.1 * count + 0.223 * work + 0.464 * max(0, values - (12 if dbl else 20)) / most
+                            + (0.05 if tt > WAVE else 0.0) + 0.1 * max(0.0, math.log2(128 / (tt * elem))))
+                    key = (round(cost, 6), order, tt)
+                    if best is None or key < best:
+                        best = key
+    return None if best is None else best[1:]
+
+
+@lru_cache(maxsize=None)
+def column_radices(N: int, elem: int, B: int) -> Optional[Tuple[Tuple[int, ...], int]]:
+    """(radices, threads per transform) of strided transforms, B of them in a workgroup: the
+    cost of balanced_plan without what only concerns contiguous rows, the smaller radices
+    first (512 = 16 32 points 8.9 us, 32 16 9.9; 320 columns, 50 MB in and out).  The idle
+    lanes are those of the workgroup's last wave: 96 points 6 16 8.7 us, 8 12 7.5."""
+    dbl = elem == 16
+    most = 16 if dbl else 32
+    if dbl and max(prime_factors(N)) > most:
+        return None
+    best = None
+    for count in (2, 3, 4, 5):
+        for rads in groupings(N, count, max(most, MAX_DIRECT_PRIME)):
+            if any(r > most and len(prime_factors(r)) > 1 for r in rads):
+                continue
+            for tt in {-(-N // (r * q)) for r in rads for q in (1, 2, 3)}:
+                values = max(slots(N, r, tt) for r in rads)
+                if tt * B > MAX_THREADS or values > max(most, max(rads)) or values < 4:
+                    continue
+                if tt * B > 512 and values > (12 if dbl else 20):  # at most 128 registers
+                    continue
+                lanes = -(-tt * B // WAVE) * WAVE / (tt * B)
+                work = sum(slots(N, r, tt) * tt for r in rads) / N * lanes
+                cost = 0.1 * count + 0.223 * work + 0.464 * max(0, values - (12 if dbl else 20)) / most
+                key = (round(cost, 6), rads[::-1], tt)
+                if best is None or key < best:
+                    best = key
+    return None if best is None else best[1:]
 
 
 def radix_plan(N: int) -> Tuple[List[int], int]:
@@ -125,10 +205,12 @@ class KernelPlan:
     NWG: int
     NWG_INNER: int
     TWREG: bool = False  # twiddles in registers, loaded with the data (a tuned option)
+    LPW: int = 0         # transforms of a wave whose last 64 - LPW TT lanes idle (0: none do)
+    CPAD: bool = False   # COLFAST: LDS positions padded by B for every first radix of them
 
     @property
     def BLOCK(self) -> int:
-        return self.B * self.TT
+        return self.B // self.LPW * WAVE if self.LPW else self.B * self.TT
 
     @property
     def fwd(self) -> List[Tuple[int, int]]:
@@ -199,10 +281,13 @@ def lookup(geom: AxisGeometry, real: str, kind: str) -> Optional[dict]:
 
 def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int] = None,
               radices: Optional[List[int]] = None, tt: Optional[int] = None,
-              need_lds: bool = False, kind: str = "fft", B_force: Optional[int] = None) -> KernelPlan:
+              need_lds: bool = False, kind: str = "fft", B_force: Optional[int] = None,
+              transposed: bool = False) -> KernelPlan:
     """Plan for ``geom``.  ``need_lds``: the kernel exchanges a full transform through
     LDS after its passes (real-FFT post-processing), so reserve B padded rows.
-    ``kind`` selects the tuned-plan entry (autotuner results / overrides) if any."""
+    ``kind`` selects the tuned-plan entry (autotuner results / overrides) if any.
+    ``transposed``: a plan of the transposed-kernel layout, whose order follows from the
+    threads and radices: these stay radix_plan's, so that stored kernels stay valid."""
     twreg = False
     if radices is None:
         hit = lookup(geom, real, kind)
@@ -211,13 +296,38 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
             B_force = hit.get("B") or B_force
             twreg = bool(hit.get("twreg", False))
     N, S, OUTER = geom.N, geom.S, geom.OUTER
-    elem = 16 if real == "double" else 8
+    dbl = real == "double"
+    elem = 16 if dbl else 8
     strided = S > 1
     if radices is None:
         if strided and N <= 32 and max(prime_factors(N) if N > 1 else [1]) <= MAX_DIRECT_PRIME:
             radices, tt = [N], 1
         else:
             radices, tt = radix_plan(N)
+            if transposed:
+                pass
+            elif strided and tt <= MAX_THREADS:
+                # whole 128-byte lines of neighbouring transforms before a second workgroup
+                # on the CU: 1000 points 32.6 us at 5 of them, 11.9 at 16; complex128 of
+                # 1024 16.9 at 4, 9.0 at 8.  Where that leaves a few large workgroups, whose
+                # own time is what the launch takes, fewer of them: 320 columns of 1000 points
+                # 10.4 us at 16, 8.2 at 8; 64 columns 10.1, 7.4 and at 4 6.7 (complex128: no gain)
+                wide = min(S, 128 // elem)
+                while wide > 1 and wide * N * elem > LDS_BYTES_MAX:
+                    wide //= 2
+                if not dbl and wide * N * elem > LDS_BYTES_TARGET:
+                    most = 16 if S * OUTER > 512 else 8 if S * OUTER > 64 else 4
+                    wide = min(wide, most)
+                hit = column_radices(N, elem, wide)
+                if hit is not None:
+                    radices, tt = hit
+                    B_force = B_force or wide
+            elif N > 32 and N not in _POW2 and tt <= MAX_THREADS:
+                hit = balanced_plan(N, elem)
+                if hit is not None:
+                    radices, tt = hit
+                    # two waves when a wave holds whole transforms, else one transform a workgroup
+                    B_force = B_force or (2 * (WAVE // tt) if tt <= WAVE else 1)
     assert tt is not None
     radices = list(radices)
     if math.prod(radices) != N:
@@ -251,18 +361,36 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
         B = max(1, min(int(B_force), S if strided else OUTER, max(1, MAX_THREADS // tt)))
         colfast = strided and B > 1
 
+    cpad = False
     if need_lds and not colfast:
         lds_elems = B * NP
     elif single_pass:
         lds_elems = 1
     elif colfast:
         lds_elems = N * B
+        padded = (N + (N - 1) // radices[0]) * B
+        # the padding against bank conflicts (512 points 10.3 -> 8.9 us) where it does not
+        # take the place of a second workgroup (complex128 of 600 points 9.9 -> 11.7 us)
+        if LDS_BYTES_MAX // (padded * elem) == LDS_BYTES_MAX // (lds_elems * elem) > 0:
+            lds_elems, cpad = padded, True
     else:
         lds_elems = B * NP
+    # A transform of at most 64 threads stays within a wave, whose exchanges need no barrier;
+    # when the threads do not divide it, the wave's last lanes idle.
+    wave_local = (not colfast) and tt <= WAVE and _wave_local_default()
+    lpw = 0
+    if transposed:
+        wave_local = wave_local and WAVE % tt == 0
+    elif wave_local and not strided and WAVE % tt:
+        lpw = WAVE // tt
+        B = max(lpw, min(-(-B // lpw), MAX_THREADS // WAVE) * lpw)
+        while B > lpw and B * NP * elem > LDS_BYTES_TARGET:
+            B -= lpw
+        if lds_elems > 1:
+            lds_elems = B * NP
     if lds_elems * elem > LDS_BYTES_MAX:
         raise ValueError(f"FFT of length {N} ({real}) needs {lds_elems * elem} bytes of LDS (max {LDS_BYTES_MAX})")
 
-    wave_local = (not colfast) and tt <= WAVE and WAVE % tt == 0 and _wave_local_default()
     if strided:
         nwg_inner = -(-S // B)
         nwg = OUTER * nwg_inner
@@ -273,7 +401,12 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
         raise ValueError("launch grid too large")
     return KernelPlan(real=real, N=N, TT=tt, B=B, S=S, OUTER=OUTER, radices=tuple(radices), COLFAST=colfast,
                       WAVE_LOCAL=wave_local, PAD_SHIFT=pad_shift, NP=NP, LDS_ELEMS=lds_elems, NWG=nwg,
-                      NWG_INNER=nwg_inner, TWREG=twreg)
+                      NWG_INNER=nwg_inner, TWREG=twreg, LPW=lpw, CPAD=cpad)
+
+
+def whole_xcds(plan: KernelPlan) -> KernelPlan:
+    """The plan with a grid of 8k workgroups (the last ones idle), as the XCD order needs."""
+    return dataclasses.replace(plan, NWG=-(-plan.NWG // 8) * 8) if plan.NWG >= 16 else plan
 
 
 def transposed_size(plan: KernelPlan) -> int:

@@ -13,7 +13,7 @@ from typing import Optional, Tuple
 from .. import dtypes as dt
 from . import hooks
 from .kernels import CompiledKernel, cfg_struct, kernel_symbol, translation_unit
-from .planner import AxisGeometry, KernelPlan, make_plan, transposed_size
+from .planner import AxisGeometry, KernelPlan, make_plan, transposed_size, whole_xcds
 from .precision import kernel_real_type
 
 
@@ -49,9 +49,9 @@ def _resolve_signal_range(signal_range, N: int) -> Tuple[int, int]:
     return s, e
 
 
-def conv_plan(buffer_shape, axis, compute_type) -> KernelPlan:
+def conv_plan(buffer_shape, axis, compute_type, transposed: bool) -> KernelPlan:
     geom = AxisGeometry.of(buffer_shape, axis)
-    return make_plan(geom, kernel_real_type(compute_type), kind="conv")
+    return make_plan(geom, kernel_real_type(compute_type), kind="conv", transposed=transposed)
 
 
 def _io_functors(args, output_map, input_map, output_type, input_type, compute, N, knum):
@@ -105,6 +105,8 @@ def make_fft_shader(buffer_shape: Tuple, axis: int = None, inverse: bool = False
     # share lines between neighbouring tiles: those tiles go to one XCD (one fetch)
     xcd = bool(input_map or output_map) or _unaligned((geom.S if geom.S > 1 else N) * output_type.item_size,
                                                       (geom.S if geom.S > 1 else N) * (input_type or output_type).item_size)
+    if xcd:
+        plan = whole_xcds(plan)
     cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=N * geom.S, sig=sig, r2c=r2c, inverse=inverse,
                      normalize=normalize, scale=1.0 / N, xcd_map=xcd)
     functors = _io_functors(args, output_map, input_map, output_type, input_type, compute, N, 1)
@@ -170,7 +172,7 @@ def make_real_rows_shader(real_shape: Tuple, inverse: bool, normalize: bool = Tr
 
 @lru_cache(maxsize=None)
 def get_transposed_size(buffer_shape: Tuple, axis: int = None, compute_type=dt.complex64) -> int:
-    return transposed_size(conv_plan(tuple(buffer_shape), axis, compute_type))
+    return transposed_size(conv_plan(tuple(buffer_shape), axis, compute_type, True))
 
 
 @lru_cache(maxsize=None)
@@ -178,7 +180,7 @@ def make_transpose_shader(buffer_shape: Tuple, axis: int = None, kernel_inner_on
                           input_type=dt.complex64, output_type=dt.complex64,
                           compute_type=dt.complex64) -> CompiledKernel:
     geom = AxisGeometry.of(buffer_shape, axis)
-    plan = conv_plan(tuple(buffer_shape), axis, compute_type)
+    plan = conv_plan(tuple(buffer_shape), axis, compute_type, True)
     from .hooks import Arg
     args = [Arg("output", "buffer", output_type, 0), Arg("input", "buffer", input_type, 1)]
     cfg = cfg_struct(plan, in_os=geom.N * geom.S, out_os=geom.N * geom.S, k_os=geom.N * geom.S, sig=(0, geom.N),
@@ -215,15 +217,17 @@ def make_convolution_shader(buffer_shape: Tuple, kernel_map=None, kernel_num: in
     compute = _compute_dtype(compute_type)
     geom = AxisGeometry.of(buffer_shape, axis)
     N = geom.N
-    plan = conv_plan(tuple(buffer_shape), axis, compute_type)
+    plan = conv_plan(tuple(buffer_shape), axis, compute_type, transposed_kernel)
     args = hooks.declare_args(output_map, input_map, kernel_map, output_type, input_type, kernel_type, conv=True)
     k_args = [a for a in args if a.role == "kernel"]
     sig = _resolve_signal_range(input_signal_range, N)
+    xcd = bool(input_map or output_map) or _unaligned(
+        (geom.S if geom.S > 1 else N) * (output_type or compute_type).item_size)
+    if xcd and not transposed_kernel:
+        plan = whole_xcds(plan)
     cfg = cfg_struct(plan, in_os=N * geom.S, out_os=N * geom.S, k_os=N * geom.S, sig=sig, r2c=False,
                      inverse=False, normalize=bool(normalize), scale=1.0 / N, knum=kernel_num,
-                     k_inner_only=kernel_inner_only, k_transposed=transposed_kernel,
-                     xcd_map=bool(input_map or output_map) or _unaligned(
-                         (geom.S if geom.S > 1 else N) * (output_type or compute_type).item_size))
+                     k_inner_only=kernel_inner_only, k_transposed=transposed_kernel, xcd_map=xcd)
     functors = _io_functors(args, output_map, input_map, output_type, input_type, compute, N, kernel_num)
     if kernel_map is not None:
         functors.append(hooks.functor_source("HookKernel", kernel_map, k_args, compute, N, writing=False,
