@@ -238,6 +238,7 @@ class CompiledKernel:
         self.source = launch_comment(self.launch_metadata(source)) + source
         self._plan_handle = None
         self._lock = threading.Lock()
+        self._buffers_only = all(a.kind == "buffer" for a in self.args)
 
     def launch_metadata(self, source: Optional[str] = None) -> Dict:
         return {"symbol": source_symbol(source if source is not None else self.source),
@@ -302,6 +303,11 @@ class CompiledKernel:
         if len(values) != len(self.args):
             raise ValueError(f"{self.name} expects {len(self.args)} arguments "
                              f"({', '.join(a.kind + ':' + a.dtype.name for a in self.args)}), got {len(values)}")
+        if self._buffers_only:  # nothing to pack
+            try:
+                return [int(v.ptr) for v in values], b""
+            except (AttributeError, TypeError):
+                pass  # refused below, with the argument
         ptrs: List[int] = []
         consts = bytearray(256)
         used = 0
@@ -330,11 +336,12 @@ class CompiledKernel:
         self.launch_raw(ptrs, consts, stream)
 
     def launch_raw(self, ptrs: Sequence[int], consts: bytes = b"", stream: Optional[int] = None) -> None:
-        h = self.handle()
-        arr = (ctypes.c_uint64 * max(1, len(ptrs)))(*ptrs)
-        cbuf = ctypes.create_string_buffer(consts, max(1, len(consts)))
-        s = rt.current_stream() if stream is None else int(stream)
-        rt.check(rt.lib().vkx_plan_exec(h, arr, len(ptrs), cbuf, len(consts), s), f"{self.name} launch")
+        # the launch copies pointers and constants, so both are passed as they are
+        n = len(ptrs)
+        rc = rt.lib().vkx_plan_exec(self._plan_handle or self.handle(), (ctypes.c_uint64 * (n or 1))(*ptrs), n, consts,
+                                    len(consts), rt.current_stream() if stream is None else int(stream))
+        if rc:
+            rt.check(rc, f"{self.name} launch")
 
     def launch_timed(self, values: Sequence, start, stop, stream: Optional[int] = None) -> None:
         """One launch whose dispatch records its own start / stop times in two

@@ -29,10 +29,10 @@ class CommandGraph:
 
     def record_kernel(self, kernel, values) -> None:
         ptrs, consts = kernel.bind(values)
-        kernel.handle()
         if self.submit_on_record:
             kernel.launch_raw(ptrs, consts)
             return
+        kernel.handle()
         # The record holds the Buffer objects themselves, not only their addresses: a
         # buffer owned by a cached plan (pair-convolution or mixed-precision scratch)
         # must outlive the plan's eviction from its cache while this graph can replay.
@@ -185,6 +185,8 @@ def global_graph() -> CommandGraph:
 
 
 def dispatch(kernel, values, graph: Optional[CommandGraph] = None) -> None:
-    if graph is not None and not isinstance(graph, CommandGraph):
+    if graph is None:
+        graph = global_graph()
+    elif not isinstance(graph, CommandGraph):
         raise ValueError("Expected a CommandGraph object for 'graph'!")
-    (graph if graph is not None else global_graph()).record_kernel(kernel, values)
+    graph.record_kernel(kernel, values)
