@@ -355,3 +355,17 @@ def test_two_launch_transform_in_a_graph():
         vd.fft.fft(other)
         vd.synchronize()
     assert O.rel_l2(other.read(0), ref) < 1e-6
+
+
+@pytest.mark.parametrize("block", [256, 512])
+def test_ragged_held_lengths_at_their_edges(block):
+    """Whole transforms in LDS where the padded copy just fits and just does not (4096 /
+    4160 points of 4224, 9920 / 9936 of 10232), single-pass and single-point ones, in place
+    (forward, then inverse)."""
+    sizes = [1, 2, 13, 16, 17, 4000, 4095, 4096, 4116, 4160, 4200, 4224, 9900, 9920, 9984, 10192, 10240]
+    parts, packed = _packed(sizes, 41)
+    buf = vd.asbuffer(packed)
+    R.RaggedFFT(sizes, block=block, classes=0, four_step=False)(buf)
+    assert _check(sizes, parts, buf.read(0)) < 1e-5
+    R.RaggedFFT(sizes, inverse=True, block=block, classes=0, four_step=False)(buf)
+    assert O.rel_l2(buf.read(0), packed) < 1e-5

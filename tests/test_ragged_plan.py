@@ -353,3 +353,25 @@ def test_class_lanes_balance_by_bytes():
     assert R.class_lanes(cs[:1], 3) == [[0]]  # empty lanes are dropped
     assert R.class_lanes([], 2) == []
     assert len(R.class_lanes(cs, 8)) == len(cs)
+
+
+def test_plan_tile_min():
+    """Lengths a workgroup cannot hold are tiled where others are anyway and they are few."""
+    assert R.plan_tile_min([9000] * 8, 512, 256) == 16384          # nothing else is tiled
+    assert R.plan_tile_min([9000, 65536], 512, 256) == R.LDS_TILE + 1
+    assert R.plan_tile_min([9000, 4099], 512, 256) == R.LDS_TILE + 1  # a tiled Bluestein length
+    assert R.plan_tile_min([9000, 1031], 512, 256) == 16384        # its power of two fits LDS
+    assert R.plan_tile_min([9000, 65536], 512, 512) == R.LDS_WHOLE_512 + 1
+    assert R.plan_tile_min([9000] * 200 + [65536], 512, 256) == 16384
+    assert R.plan_tile_min([65536] * 600 + [9000], 512, 256) == R.TILE_MIN_DIRECT
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 5, 7, 13, 16, 97, 255, 256, 4095, 4224, 65535, 2 ** 21 + 1])
+def test_division_by_reciprocal_is_exact(d):
+    """The kernel's Div: float32 product, truncated, put right by at most one, below 2^22."""
+    edges = np.arange(0, 2 ** 22, d, dtype=np.int64)[:20000]
+    j = np.unique(np.clip(np.concatenate([edges, edges - 1, edges + 1, np.arange(2 ** 22 - 3000, 2 ** 22),
+                                          np.random.default_rng(d).integers(0, 2 ** 22, 50000)]), 0, 2 ** 22 - 1))
+    q = (j.astype(np.float32) * (np.float32(1) / np.float32(d))).astype(np.int64)
+    m = j - q * d
+    assert np.array_equal(q + (m >= d) - (m < 0), j // d)

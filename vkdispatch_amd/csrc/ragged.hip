@@ -51,81 +51,58 @@ static_assert(sizeof(RTask) == 128, "RTask layout");
 constexpr int kLdsBuf = 4096 + 128;
 constexpr int kLdsBig = 10232;  // 2 x 10232 x 8 B + the queue slot fit in 160 KB
 
-template <int R, int DIR>
-__device__ __forceinline__ void bfly(const c64* __restrict__ src, c64* __restrict__ dst, const c64* __restrict__ tw,
-                                     int n, int count, int ns, float scale, int pitch) {
-  const int W = n / R;
-  const int total = W * count;
-  for (int jj = threadIdx.x; jj < total; jj += blockDim.x) {
-    const int c = jj / W;
-    const int j = jj - c * W;
-    const int off = c * pitch;
-    const int k = j % ns;
-    c64 v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = src[off + j + r * W];
-    if (ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        c64 w = tw[(ns - 1) + (r - 1) * ns + k];
-        if (DIR > 0) w.y = -w.y;
-        v[r] = vkx::cmul(v[r], w);
-      }
-    }
-    vkx::DFT<R, DIR>::run(v);
-    const int base = off + (j / ns) * ns * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) dst[base + r * ns] = v[r] * scale;
-  }
+// Pointers held as integers in a task: formed in the global address space, so that they
+// compile to global_ and not flat_ accesses (which also wait for LDS).
+template <class T> __device__ __forceinline__ T* gptr(unsigned long long a) {
+  return (T*)(__attribute__((address_space(1))) T*)a;
 }
 
-template <int DIR>
-__device__ void pass_dispatch(int R, const c64* src, c64* dst, const c64* tw, int n, int count, int ns, float scale,
-                              int pitch) {
-  switch (R) {
-    case 2: bfly<2, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 3: bfly<3, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 4: bfly<4, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 5: bfly<5, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 6: bfly<6, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 7: bfly<7, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 8: bfly<8, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 9: bfly<9, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 10: bfly<10, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 11: bfly<11, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 12: bfly<12, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 13: bfly<13, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    case 16: bfly<16, DIR>(src, dst, tw, n, count, ns, scale, pitch); break;
-    default: break;  // the host planner emits only the radices above
+// Division by a value the workgroup shares: by its reciprocal, put right by at most one
+// (the numerators are below 2^22, `exact` for larger), 7 instructions instead of 25.
+struct Div {
+  int d;
+  float r;
+  bool exact;
+  __device__ __forceinline__ Div(int d_, int top) : d(d_), r(1.0f / (float)d_), exact(top >= (1 << 22)) {}
+  __device__ __forceinline__ int operator()(int j) const {
+    if (exact) return j / d;
+    int q = (int)((float)j * r);
+    const int m = j - q * d;
+    q += m >= d ? 1 : 0;
+    q -= m < 0 ? 1 : 0;
+    return q;
   }
-}
+};
 
 // One pass of a single length-n transform from global to global memory whose output
 // runs (ns consecutive elements) are shorter than a cache line: each round takes whole
 // groups of ns butterflies, so its R outputs per butterfly fill one contiguous range,
 // which goes through LDS (`stage`, padded one element per 16) and out in full lines.
-// Every thread runs the same rounds (the barriers are uniform).
-template <int R, int DIR>
+// Every thread runs the same rounds (the barriers are uniform).  Forward; an inverse
+// transform conjugates on its first load and its last store (cin, cout).
+template <int R>
 __device__ __forceinline__ void bfly_staged(const c64* __restrict__ src, c64* __restrict__ dst,
-                                            const c64* __restrict__ tw, int n, int ns, float scale, c64* stage) {
+                                            const c64* __restrict__ tw, int n, int ns, bool cin, bool cout,
+                                            float scale, c64* stage) {
   const int W = n / R;  // a multiple of ns
   const int C = (int)(blockDim.x / ns) * ns;
+  const Div by_ns(ns, W);
   for (int j0 = 0; j0 < W; j0 += C) {
     const int j = j0 + (int)threadIdx.x;
     if ((int)threadIdx.x < C && j < W) {
-      const int k = j % ns;
+      const int k = j - by_ns(j) * ns;
       c64 v[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = src[j + r * W];
+      if (cin) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r].y = -v[r].y;
+      }
       if (ns > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) {
-          c64 w = tw[(ns - 1) + (r - 1) * ns + k];
-          if (DIR > 0) w.y = -w.y;
-          v[r] = vkx::cmul(v[r], w);
-        }
+        for (int r = 1; r < R; ++r) v[r] = vkx::cmul(v[r], tw[(ns - 1) + (r - 1) * ns + k]);
       }
-      vkx::DFT<R, DIR>::run(v);
+      vkx::DFT<R, -1>::run(v);
       const int q0 = (j - j0 - k) * R + k;  // output position relative to j0 R
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -135,98 +112,43 @@ __device__ __forceinline__ void bfly_staged(const c64* __restrict__ src, c64* __
     }
     __syncthreads();
     const int cnt = min(C, W - j0) * R;
-    for (int i = threadIdx.x; i < cnt; i += blockDim.x) dst[j0 * R + i] = stage[i + (i >> 4)];
+    for (int i = threadIdx.x; i < cnt; i += blockDim.x) {
+      c64 v = stage[i + (i >> 4)];
+      if (cout) v.y = -v.y;
+      dst[j0 * R + i] = v;
+    }
     __syncthreads();
   }
 }
 
-template <int DIR>
-__device__ void pass_dispatch_staged(int R, const c64* src, c64* dst, const c64* tw, int n, int ns, float scale,
-                                     c64* stage) {
+__device__ __forceinline__ void pass_staged(int R, const c64* src, c64* dst, const c64* tw, int n, int ns, bool cin, bool cout,
+                            float scale, c64* stage) {
   switch (R) {
-    case 2: bfly_staged<2, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 3: bfly_staged<3, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 4: bfly_staged<4, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 5: bfly_staged<5, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 6: bfly_staged<6, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 7: bfly_staged<7, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 8: bfly_staged<8, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 9: bfly_staged<9, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 10: bfly_staged<10, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 11: bfly_staged<11, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 12: bfly_staged<12, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 13: bfly_staged<13, DIR>(src, dst, tw, n, ns, scale, stage); break;
-    case 16: bfly_staged<16, DIR>(src, dst, tw, n, ns, scale, stage); break;
+    case 2: bfly_staged<2>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 3: bfly_staged<3>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 4: bfly_staged<4>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 5: bfly_staged<5>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 6: bfly_staged<6>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 7: bfly_staged<7>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 8: bfly_staged<8>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 9: bfly_staged<9>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 10: bfly_staged<10>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 11: bfly_staged<11>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 12: bfly_staged<12>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 13: bfly_staged<13>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
+    case 16: bfly_staged<16>(src, dst, tw, n, ns, cin, cout, scale, stage); break;
     default: break;  // the host planner emits only the radices above
   }
 }
 
-__device__ void copy_elems(const c64* src, c64* dst, int total) {
-  for (int i = threadIdx.x; i < total; i += blockDim.x) dst[i] = src[i];
-}
-
-// Stockham pass list from src to dst; T0/T1 are ping-pong buffers distinct from
-// dst (T1 may alias src: src is only read by pass 0).  Ends with a barrier.
-__device__ void run_fft(const c64* src, c64* dst, c64* T0, c64* T1, const RTask& t, int n, const int* radix,
-                        int npass, int dir, float scale) {
-  const c64* tw = reinterpret_cast<const c64*>(t.tw);
-  if (npass == 1 && src == dst) {  // single pass in place: stage through T0
-    copy_elems(src, T0, n * t.count);
-    __syncthreads();
-    src = T0;
-    T0 = T1;
-  }
-  int ns = 1;
-  const c64* in = src;
-  for (int p = 0; p < npass; ++p) {
-    const bool last = p == npass - 1;
-    c64* out = last ? dst : ((p & 1) ? T1 : T0);
-    if (dir > 0) pass_dispatch<1>(radix[p], in, out, tw, n, t.count, ns, last ? scale : 1.0f, n);
-    else pass_dispatch<-1>(radix[p], in, out, tw, n, t.count, ns, last ? scale : 1.0f, n);
-    __syncthreads();
-    ns *= radix[p];
-    in = out;
-  }
-}
-
-// The same pass list for one transform (count 1) through global memory: the passes
-// alternate between T0 and dst, so that the last one lands in dst and a transform
-// touches one scratch buffer of its length instead of two.  In place (src == dst), a
-// first pass that would write dst goes to T1.  Passes whose output runs are shorter
-// than 16 elements (128 bytes) are written through `stage` (LDS, room for
-// blockDim.x * 17 elements).  Needs npass >= 2.  Ends with a barrier.
-__device__ void run_fft_global(const c64* src, c64* dst, c64* T0, c64* T1, c64* stage, const RTask& t, int n,
-                               const int* radix, int npass, int dir, float scale) {
-  const c64* tw = reinterpret_cast<const c64*>(t.tw);
-  int ns = 1;
-  const c64* in = src;
-  for (int p = 0; p < npass; ++p) {
-    const bool last = p == npass - 1;
-    c64* out = ((npass - 1 - p) & 1) ? T0 : dst;
-    if (p == 0 && out == src) out = T1;
-    const float sc = last ? scale : 1.0f;
-    if (ns < 16) {
-      if (dir > 0) pass_dispatch_staged<1>(radix[p], in, out, tw, n, ns, sc, stage);
-      else pass_dispatch_staged<-1>(radix[p], in, out, tw, n, ns, sc, stage);
-    } else {
-      if (dir > 0) pass_dispatch<1>(radix[p], in, out, tw, n, 1, ns, sc, n);
-      else pass_dispatch<-1>(radix[p], in, out, tw, n, 1, ns, sc, n);
-    }
-    __syncthreads();
-    ns *= radix[p];
-    in = out;
-  }
-}
-
-// exp(-2 pi i p / L) for 0 <= p < 2^31 (the host keeps tiled lengths <= 2^18)
+// exp(-2 pi i p / L) for 0 <= p < L (the host keeps tiled lengths <= 2^18)
 __device__ __forceinline__ c64 twiddle_L(int p, int L) {
-  const int q = p % L;
   float s, c;
-  sincospif(2.0f * (float)q / (float)L, &s, &c);
+  sincospif(2.0f * (float)p / (float)L, &s, &c);
   return c64{c, -s};
 }
 
-// ---- tiles of a long transform ---------------------------------------------------
+// ---- passes ------------------------------------------------------------------------
 // A transform of length L = n1 n2 (x[j1 n2 + j2]) runs as work items of two kinds:
 // column tiles (length-n1 transforms over j1 for a run of columns j2, times
 // W_L^(k1 j2), stored row-major y[k1 n2 + j2]) and row tiles (length-n2 transforms
@@ -234,16 +156,35 @@ __device__ __forceinline__ c64 twiddle_L(int p, int L) {
 // Stockham pass; inverse transforms conjugate on the way in and out.  Pass 0 reads
 // global memory and the last pass writes it, the passes between ping-pong in LDS at
 // pitch n + 1, so a tile crosses HBM once each way.  Threads take consecutive columns
-// (rows) where that makes the global access a run of the tile's width.
+// (rows) where that makes the global access a run of the tile's width.  A whole
+// transform that fits is one such row.
+//
+// All of it is inlined into the kernel, one copy of each pass for a kind of source and
+// a kind of destination: the task's fields stay scalars and nothing goes through the
+// stack.  As calls on a task copied to the stack the kernel took 248 registers and 240
+// bytes of scratch a lane, and every radix was a lane's own: 96 registers now; 1194 smooth
+// lengths of 64 to 65536 points (169 MB in and out) tiled 262 -> 177 us, mixes of 300 /
+// 1000 / 4096 transforms 221 -> 163, 358 -> 288 and 716 -> 675 us.
 
 // Store functors with kRun take a butterfly's R outputs at once (run<R>), the others
 // one element at a time (st).
-struct LdsIO {  // element (c, j) of an LDS tile
+struct LdsIO {  // element (c, j) of an LDS tile; pad: one element more for every 2^pad of them
   static constexpr bool kRun = false;
   c64* p;
+  int pitch, pad;
+  __device__ __forceinline__ c64 ld(int c, int j) const { return p[c * pitch + j + (j >> pad)]; }
+  __device__ __forceinline__ void st(int c, int j, c64 v) const { p[c * pitch + j + (j >> pad)] = v; }
+};
+
+struct RowLoad {  // element j of row c at `pitch` from src
+  const c64* src;
   int pitch;
-  __device__ __forceinline__ c64 ld(int c, int j) const { return p[c * pitch + j]; }
-  __device__ __forceinline__ void st(int c, int j, c64 v) const { p[c * pitch + j] = v; }
+  bool conj;
+  __device__ __forceinline__ c64 ld(int c, int j) const {
+    c64 v = src[c * pitch + j];
+    if (conj) v.y = -v.y;
+    return v;
+  }
 };
 
 struct ColLoad {  // element j1 of column c0 + c: x[j1 n2 + c0 + c]
@@ -268,7 +209,7 @@ struct ColStore {  // y[k1 n2 + j2] = v W_L^(k1 j2), j2 = c0 + c
   static constexpr bool kRun = true;
   c64* dst;
   int n2, c0, L;
-  // outputs k1 = base + r ns of one butterfly (k1 j2 < n1 n2 = L): the twiddle is
+  // outputs k1 = base + r ns of one butterfly (k1 j2 and ns j2 < n1 n2 = L): the twiddle is
   // evaluated for every fourth r and stepped by W_L^(ns j2) in between
   template <int R>
   __device__ __forceinline__ void run(int c, int base, int ns, const c64 (&v)[R]) const {
@@ -284,20 +225,14 @@ struct ColStore {  // y[k1 n2 + j2] = v W_L^(k1 j2), j2 = c0 + c
   }
 };
 
-struct RowLoad {  // element j2 of row r0 + t: y[(r0 + t) n2 + j2]
-  const c64* src;
-  int n2, r0;
-  __device__ __forceinline__ c64 ld(int t, int j2) const { return src[(r0 + t) * n2 + j2]; }
-};
-
-struct RowStore {  // X[k] with k = r0 + t + n1 k2
+struct RowStore {  // X[k] with k = r0 + t pitch + n1 k2
   static constexpr bool kRun = false;
   c64* dst;
   const c64* aux;  // mode 2: Bluestein kernel spectrum; mode 3: chirp
-  int n1, r0, m, nvalid, mode, inv;
+  int pitch, n1, r0, m, nvalid, mode, inv;
   float scale;
   __device__ __forceinline__ void st(int t, int k2, c64 v) const {
-    const int k = r0 + t + n1 * k2;
+    const int k = r0 + t * pitch + n1 * k2;
     if (mode == 0) {  // v (conjugated for an inverse transform) times scale
       if (inv) v.y = -v.y;
       dst[k] = v * scale;
@@ -326,16 +261,11 @@ template <int R, class Ld, class St>
 __device__ __forceinline__ void bfly_io(const c64* __restrict__ tw, int W, int count, int ns, bool cfast,
                                         const Ld& ld, const St& st) {
   const int total = W * count;
+  const Div by(cfast ? count : W, total), by_ns(ns, total);
   for (int jj = threadIdx.x; jj < total; jj += blockDim.x) {
-    int c, j;
-    if (cfast) {
-      j = jj / count;
-      c = jj - j * count;
-    } else {
-      c = jj / W;
-      j = jj - c * W;
-    }
-    const int k = j % ns;
+    const int q = by(jj), m = jj - q * by.d;
+    const int c = cfast ? m : q, j = cfast ? q : m;
+    const int jn = by_ns(j), k = j - jn * ns;
     c64 v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = ld.ld(c, j + r * W);
@@ -344,7 +274,7 @@ __device__ __forceinline__ void bfly_io(const c64* __restrict__ tw, int W, int c
       for (int r = 1; r < R; ++r) v[r] = vkx::cmul(v[r], tw[(ns - 1) + (r - 1) * ns + k]);
     }
     vkx::DFT<R, -1>::run(v);
-    const int base = (j / ns) * ns * R + k;
+    const int base = jn * ns * R + k;
     if constexpr (St::kRun) {
       st.template run<R>(c, base, ns, v);
     } else {
@@ -355,7 +285,8 @@ __device__ __forceinline__ void bfly_io(const c64* __restrict__ tw, int W, int c
 }
 
 template <class Ld, class St>
-__device__ void pass_io(int R, const c64* tw, int n, int count, int ns, bool cfast, const Ld& ld, const St& st) {
+__device__ __forceinline__ void pass_io(int R, const c64* tw, int n, int count, int ns, bool cfast, const Ld& ld,
+                                        const St& st) {
   const int W = n / R;
   switch (R) {
     case 2: bfly_io<2>(tw, W, count, ns, cfast, ld, st); break;
@@ -375,114 +306,162 @@ __device__ void pass_io(int R, const c64* tw, int n, int count, int ns, bool cfa
   }
 }
 
-// `count` length-n transforms, global -> (LDS ping-pong at `pitch`) -> global.  A tile
-// of up to two passes uses only lds0 (and may extend over lds1); longer pass lists
-// alternate lds0 / lds1.  cfast0 / cfast: thread order of pass 0 / the other passes.
-template <class GLd, class GSt>
-__device__ void tile_fft(const c64* tw, int n, int count, int pitch, const int* radix, int npass, c64* lds0,
-                         c64* lds1, const GLd& gld, const GSt& gst, bool cfast0, bool cfast) {
-  int ns = 1;
-  for (int p = 0; p < npass; ++p) {
-    const bool first = p == 0, last = p == npass - 1;
-    const LdsIO src{(p & 1) ? lds0 : lds1, pitch};  // written by pass p - 1
-    const LdsIO dst{(p & 1) ? lds1 : lds0, pitch};
-    const bool cf = first ? cfast0 : cfast;
-    if (first && last) pass_io(radix[p], tw, n, count, ns, cf, gld, gst);
-    else if (first) pass_io(radix[p], tw, n, count, ns, cf, gld, dst);
-    else if (last) pass_io(radix[p], tw, n, count, ns, cf, src, gst);
-    else pass_io(radix[p], tw, n, count, ns, cf, src, dst);
-    if (!last) __syncthreads();
-    ns *= radix[p];
-  }
-}
-
 // Item kinds (task bits 16-19); bit 20: conjugate (inverse direct transform).
 enum : int { kWhole = 0, kCol = 1, kRow = 2, kBlueCol = 3, kBlueRow = 4, kBlueOut = 5 };
 
-__device__ void run_tile(const RTask& t, int kind, c64* lds0, c64* lds1) {
+// `count` length-n transforms, global -> (LDS ping-pong) -> global: a whole transform
+// that fits or a tile.  Up to two passes use only lds0 (and may extend over lds1); longer
+// pass lists alternate lds0 / lds1.
+__device__ __forceinline__ void run_lds(const RTask& t, int kind, c64* lds, int cap) {
+  const int np1 = (t.npass >> 8) & 0xff, cj = (t.npass >> 20) & 1;
+  const bool whole = kind == kWhole, cols = kind == kCol || kind == kBlueCol;
   const int L = t.m ? t.m : t.n;
-  const int npass = t.npass & 0xff, np1 = (t.npass >> 8) & 0xff;
-  const int cj = (t.npass >> 20) & 1;
-  int n1 = 1;
+  int n1 = 1, p0 = 0, npass = t.npass & 0xff;
   for (int p = 0; p < np1; ++p) n1 *= t.radix[p];
   const int n2 = L / n1;
-  const c64* tw = reinterpret_cast<const c64*>(t.tw);
-  const c64* in = reinterpret_cast<const c64*>(t.in);
-  c64* out = reinterpret_cast<c64*>(t.out);
-  if (kind == kCol || kind == kBlueCol) {
+  const c64* tw = gptr<const c64>(t.tw);
+  const c64* in = gptr<const c64>(t.in);
+  c64* out = gptr<c64>(t.out);
+  if (cols) {
+    npass = np1;
+  } else if (!whole) {
+    p0 = np1;
+    npass -= np1;
+    tw += n1 - 1;
+  }
+  const int n = cols ? n1 : n2, count = t.count;  // whole: n1 = 1, n2 = n
+  const int pitch = whole ? n : n + 1, total = n * count;
+  // a whole transform's first writes are its radix apart: one element more for every 32
+  // keeps them off each other's banks, where there is room
+  const LdsIO even{lds, pitch, whole && count == 1 && total + (total >> 5) <= cap ? 5 : 31};
+  const LdsIO odd{lds + cap, pitch, even.pad};
+
+  if (npass == 0) return;  // a single point, in place
+  const int R0 = t.radix[p0];
+  if (cols) {
     // direct columns conjugate the data of an inverse transform (bit 20); Bluestein
     // columns conjugate the chirp of an inverse transform
     const bool blue = kind == kBlueCol;
-    const ColLoad ld{in, reinterpret_cast<const c64*>(t.chirp), n2, t.tile0, t.n, blue ? 2 : 0,
-                     blue ? t.inverse : cj};
-    const ColStore st{out, n2, t.tile0, L};
-    tile_fft(tw, n1, t.count, n1 + 1, t.radix, np1, lds0, lds1, ld, st, true, true);
+    const ColLoad ld{in, gptr<const c64>(t.chirp), n2, t.tile0, t.n, blue ? 2 : 0, blue ? t.inverse : cj};
+    pass_io(R0, tw, n, count, 1, true, ld, even);
   } else {
-    const int np2 = npass - np1;
-    const RowLoad ld{in, n2, t.tile0};
-    const int mode = kind == kRow ? 0 : (kind == kBlueRow ? 2 : 3);
-    const c64* aux = reinterpret_cast<const c64*>(kind == kBlueRow ? t.bspec : t.chirp);
-    const RowStore st{out, aux, n1, t.tile0, L, t.n, mode, kind == kRow ? cj : t.inverse, t.scale};
-    tile_fft(tw + (n1 - 1), n2, t.count, n2 + 1, t.radix + np1, np2, lds0, lds1, ld, st, np2 == 1, true);
+    const RowLoad ld{in + (whole ? 0 : t.tile0 * n2), n, whole && t.inverse};
+    pass_io(R0, tw, n, count, 1, false, ld, even);
+  }
+  __syncthreads();
+  int ns = R0, p = 1;
+  for (; p < npass - 1; ++p) {
+    const int R = t.radix[p0 + p];
+    const LdsIO src{(p & 1) ? even.p : odd.p, pitch, even.pad}, dst{(p & 1) ? odd.p : even.p, pitch, even.pad};
+    pass_io(R, tw, n, count, ns, !whole, src, dst);
+    __syncthreads();
+    ns *= R;
+  }
+  const LdsIO src{(p & 1) ? even.p : odd.p, pitch, even.pad};
+  if (cols) {
+    const ColStore st{out, n2, t.tile0, L};
+    if (npass == 1) {  // one pass: as it is
+      for (int i = threadIdx.x; i < total; i += blockDim.x) {
+        const c64 v[1] = {src.ld(i % count, i / count)};
+        st.run<1>(i % count, i / count, 1, v);
+      }
+    } else {
+      pass_io(t.radix[p0 + p], tw, n, count, ns, true, src, st);
+    }
+  } else {
+    const int mode = whole || kind == kRow ? 0 : (kind == kBlueRow ? 2 : 3);
+    const RowStore st{out, gptr<const c64>(kind == kBlueRow ? t.bspec : t.chirp), whole ? n : 1, n1,
+                      whole ? 0 : t.tile0, L, t.n, mode, kind == kRow ? cj : t.inverse, t.scale};
+    if (npass == 1) {
+      for (int i = threadIdx.x; i < total; i += blockDim.x) st.st(i % count, i / count, src.ld(i % count, i / count));
+    } else {
+      pass_io(t.radix[p0 + p], tw, n, count, ns, !whole, src, st);
+    }
   }
 }
 
-// lds_cap: elements of each of the two LDS buffers
-__device__ void run_task(const RTask& t, c64* lds0, c64* lds1, int lds_cap, c64* scr) {
-  const c64* in = reinterpret_cast<const c64*>(t.in);
-  c64* out = reinterpret_cast<c64*>(t.out);
-  const int dir = t.inverse ? 1 : -1;
-  const int npass = t.npass & 0xff;
-  if (t.m == 0) {
-    const int total = t.n * t.count;
-    if (total <= lds_cap) {
-      run_fft(in, out, lds0, lds1, t, t.n, t.radix, npass, dir, t.scale);
-    } else if (npass < 2 || t.count != 1) {
-      run_fft(in, out, scr, scr + total, t, t.n, t.radix, npass, dir, t.scale);
-    } else {
-      run_fft_global(in, out, scr, scr + total, lds0, t, t.n, t.radix, npass, dir, t.scale);
-    }
-    return;
-  }
+// A whole transform through global memory: one forward pass list (conjugated on the way in
+// and out of an inverse one), or for a Bluestein length two with the chirp spectrum between
+// them, in this workgroup's scratch slice `scr`.  The passes alternate between T0 and the
+// destination, so that the last one lands there and a transform touches one scratch buffer
+// of its length; in place, a first pass that would write the destination goes to T1 (a
+// single pass too, copied back).  Passes of one transform whose output runs are shorter
+// than 16 elements (128 bytes) are written through `stage` (LDS, room for blockDim.x * 17
+// elements).
+__device__ __forceinline__ void run_global(const RTask& t, c64* stage, c64* scr) {
   // Bluestein: X[k] = w[k] * sum_j (x[j] w[j]) conj(w[k-j]),  w[j] = exp(-i pi j^2 / n)
-  const int n = t.n, m = t.m;
-  const c64* w = reinterpret_cast<const c64*>(t.chirp);
-  const c64* bs = reinterpret_cast<const c64*>(t.bspec);
+  const int m = t.m, n = m ? m : t.n, per = m ? 1 : t.count, npass = t.npass & 0xff;
+  const c64* tw = gptr<const c64>(t.tw);
+  const c64* w = gptr<const c64>(t.chirp);
+  const c64* bs = gptr<const c64>(t.bspec);
   c64* S0 = scr;
-  c64* S1 = scr + m;
-  c64* S2 = scr + 2 * m;
-  for (int c = 0; c < t.count; ++c) {
-    const c64* xin = in + (long long)c * n;
-    c64* xout = out + (long long)c * n;
-    for (int j = threadIdx.x; j < m; j += blockDim.x) {
-      c64 v{0.f, 0.f};
-      if (j < n) {
-        c64 ww = w[j];
+  c64* S1 = scr + (long long)n * per;
+  c64* S2 = scr + 2ll * n * per;
+  for (int c = 0; c < (m ? t.count : 1); ++c) {
+    const c64* xin = gptr<const c64>(t.in) + (long long)c * t.n;
+    c64* xout = gptr<c64>(t.out) + (long long)c * t.n;
+    if (m) {
+      for (int j = threadIdx.x; j < m; j += blockDim.x) {
+        c64 v{0.f, 0.f};
+        if (j < t.n) {
+          c64 ww = w[j];
+          if (t.inverse) ww.y = -ww.y;
+          v = vkx::cmul(xin[j], ww);
+        }
+        S0[j] = v;
+      }
+      __syncthreads();
+    }
+    for (int half = 0; half < (m ? 2 : 1); ++half) {
+      // direct: x -> X by S0, S1; Bluestein: S0 -> S1 by S2, S0, then S1 -> S0 by S2, S1
+      const c64* src = m ? (half ? S1 : S0) : xin;
+      c64* dst = m ? (half ? S0 : S1) : xout;
+      c64* T0 = m ? S2 : S0;
+      c64* T1 = m ? (half ? S1 : S0) : S1;
+      const bool inverse = m ? half == 1 : t.inverse != 0;
+      const float scale = m ? (half ? 1.0f / (float)m : 1.0f) : t.scale;
+      int ns = 1;
+      for (int p = 0; p < npass; ++p) {
+        const bool last = p == npass - 1, cin = inverse && p == 0, cout = inverse && last;
+        c64* to = ((npass - 1 - p) & 1) ? T0 : dst;
+        if (p == 0 && to == src) to = T1;
+        const float sc = last ? scale : 1.0f;
+        const int R = t.radix[p];
+        if (ns < 16 && per == 1) {
+          pass_staged(R, src, to, tw, n, ns, cin, cout, sc, stage);
+        } else {
+          const RowLoad ld{src, n, cin};
+          const RowStore st{to, w, n, 1, 0, n, n, 0, cout, sc};
+          pass_io(R, tw, n, per, ns, false, ld, st);
+        }
+        __syncthreads();
+        ns *= R;
+        src = to;
+      }
+      if (npass > 0 && src != dst) {
+        for (int i = threadIdx.x; i < n * per; i += blockDim.x) dst[i] = src[i];
+        __syncthreads();
+      }
+      if (m && half == 0) {
+        for (int j = threadIdx.x; j < m; j += blockDim.x) {
+          c64 b = bs[j];
+          if (t.inverse) {  // spectrum of conj(b) for the inverse chirp: B_inv[k] = conj(B[-k])
+            b = bs[(m - j) & (m - 1)];
+            b.y = -b.y;
+          }
+          S1[j] = vkx::cmul(S1[j], b);
+        }
+        __syncthreads();
+      }
+    }
+    if (m) {
+      for (int k = threadIdx.x; k < t.n; k += blockDim.x) {
+        c64 ww = w[k];
         if (t.inverse) ww.y = -ww.y;
-        v = vkx::cmul(xin[j], ww);
+        xout[k] = vkx::cmul(S0[k], ww) * t.scale;
       }
-      S0[j] = v;
+      __syncthreads();
     }
-    __syncthreads();
-    RTask sub = t;
-    sub.count = 1;
-    run_fft(S0, S1, S2, S0, sub, m, t.radix, npass, -1, 1.0f);
-    for (int j = threadIdx.x; j < m; j += blockDim.x) {
-      c64 b = bs[j];
-      if (t.inverse) {  // spectrum of conj(b) for the inverse chirp: B_inv[k] = conj(B[-k])
-        b = bs[(m - j) & (m - 1)];
-        b.y = -b.y;
-      }
-      S1[j] = vkx::cmul(S1[j], b);
-    }
-    __syncthreads();
-    run_fft(S1, S0, S2, S1, sub, m, t.radix, npass, 1, 1.0f / (float)m);
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-      c64 ww = w[k];
-      if (t.inverse) ww.y = -ww.y;
-      xout[k] = vkx::cmul(S0[k], ww) * t.scale;
-    }
-    __syncthreads();
   }
 }
 
@@ -516,15 +495,20 @@ __global__ void __launch_bounds__(512) ragged_kernel(const RTask* __restrict__ t
   __shared__ int task_id;
   c64* scr = scratch + (long long)blockIdx.x * scratch_per_wg;
   for (;;) {
+    // The task before is done with LDS and task_id is read.  The barrier also keeps the
+    // branch of thread 0 that ends a tile (its counter) apart from the one that fetches:
+    // joined by the compiler, the other lanes of its wave would go round without it.
+    __syncthreads();
     if (threadIdx.x == 0) task_id = atomicAdd(&ctr[0], 1);
     __syncthreads();
-    const int id = task_id;
-    __syncthreads();
+    const int id = __builtin_amdgcn_readfirstlane(task_id);
     if (id >= ntasks) break;
-    const RTask t = tasks[id];
+    // read through the constant address space: the task's fields are scalars, so pass
+    // loops, radix switches and divisors are the wave's and not each lane's
+    const RTask& t = *(const RTask*)(__attribute__((address_space(4))) const RTask*)(tasks + id);
     const int kind = (t.npass >> 16) & 0xf;
-    if (kind == kWhole) {
-      run_task(t, lds, lds + CAP, CAP, scr);
+    if (kind == kWhole && (t.m != 0 || t.n * t.count > CAP)) {
+      run_global(t, lds, scr);
       continue;
     }
     if (t.dep >= 0) {
@@ -532,7 +516,7 @@ __global__ void __launch_bounds__(512) ragged_kernel(const RTask* __restrict__ t
       __syncthreads();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
-    run_tile(t, kind, lds, lds + CAP);
+    run_lds(t, kind, lds, CAP);
     if (t.done >= 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __syncthreads();

@@ -67,6 +67,7 @@ CONJ = 1 << 20
 
 LDS_PINGPONG = 4096
 LDS_TILE = 4096 + 128  # complex64 elements of one LDS buffer (a tile at pitch n + 1)
+LDS_WHOLE_512 = 10232  # whole transforms that workgroups of 512 threads hold (they take all of the LDS)
 FOUR_STEP_MAX = 512  # longest four-step factor: tiles of >= 8 padded columns fit one LDS buffer
 TILE_MIN_DIRECT = 1 << 17  # direct lengths from here on are tiled (shorter ones run whole on one workgroup)
 DIRECT_PRIMES = (2, 3, 5, 7, 11, 13)
@@ -143,6 +144,23 @@ def auto_tile_min(sizes: Sequence[int], resident_wgs: int) -> int:
     then cost less than the tiles' two extra passes)."""
     n_long = sum(1 for n in sizes if n >= 16384 and is_direct(int(n)))
     return 16384 if n_long < resident_wgs else TILE_MIN_DIRECT
+
+
+def plan_tile_min(sizes: Sequence[int], resident_wgs: int, block: int) -> int:
+    """auto_tile_min of the transforms left to the persistent kernel.  Where others are tiled
+    anyway, a few lengths below it that a workgroup cannot hold in LDS are tiled too: alone
+    it takes them through global memory pass by pass, 40 to 75 us that the batch waits for
+    (mixes of 150 and 300 transforms 168 -> 120 and 194 -> 160 us; above 2^20 points the
+    workgroups have enough of them: 300 x 14406 points 87 us whole, 107 tiled; and without
+    other tiles 8 x 9000 points 37 us either way, 8 x 5000 28 and 31)."""
+    at = auto_tile_min(sizes, resident_wgs)
+    held = (LDS_WHOLE_512 if block == 512 else LDS_TILE) + 1
+    if at == TILE_MIN_DIRECT:
+        return at
+    direct = [int(n) for n in sizes if is_direct(int(n))]
+    others = max(direct, default=0) >= at or any(
+        not is_direct(int(n)) and bluestein_length(int(n)) > LDS_PINGPONG for n in sizes)
+    return held if others and sum(n for n in direct if held <= n < at) < 1 << 20 else at
 
 
 def tile_log2_width(n: int, npass: int = 3) -> int:
@@ -469,9 +487,6 @@ class RaggedFFT:
         self.max_radix = int(max_radix)
         self.spin_limit = int(spin_limit)
         dev = rt.ensure_device()
-        if tile_min is None:
-            tile_min = auto_tile_min(self.sizes, 2 * int(dev.compute_units))
-        self.tile_min = int(tile_min)
         self.sync = sync
         self.classes = int(classes)
         if int(class_streams) < 1:
@@ -483,6 +498,9 @@ class RaggedFFT:
         rest = np.ones(len(self.sizes), bool)
         for idx in list(groups.values()) + list(bgroups.values()):
             rest[idx] = False
+        if tile_min is None:
+            tile_min = plan_tile_min(self.sizes[rest], 2 * int(dev.compute_units), self.block_first)
+        self.tile_min = int(tile_min)
         self._classes = [BlueClass(m, self.sizes[idx], self.offsets[idx], self.inverse, self.normalize, self.max_radix)
                          for m, idx in sorted(bgroups.items(), reverse=True)]
         self._classes += [LengthClass(L, self.offsets[idx], self.inverse, self.normalize)
