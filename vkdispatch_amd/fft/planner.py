@@ -91,12 +91,18 @@ def balanced_plan(N: int, elem: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     return None if best is None else best[1:]
 
 
+UNEVEN_LDS = 44 * 1024  # up to here enough workgroups share a CU to even its four SIMDs out
+
+
 @lru_cache(maxsize=None)
 def column_radices(N: int, elem: int, B: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     """(radices, threads per transform) of strided transforms, B of them in a workgroup: the
     cost of balanced_plan without what only concerns contiguous rows, the smaller radices
     first (512 = 16 32 points 8.9 us, 32 16 9.9; 320 columns, 50 MB in and out).  The idle
-    lanes are those of the workgroup's last wave: 96 points 6 16 8.7 us, 8 12 7.5."""
+    lanes are those of the workgroup's last wave: 96 points 6 16 8.7 us, 8 12 7.5.  Two or
+    three large workgroups on a CU want waves for all four SIMDs: 480 points of 24 threads
+    (6 waves) 11.1 us, of 16 (4 waves) 9.2, convolved 18.2 and 15.5; complex128 432 points
+    5 waves 10.8, 7 waves 8.2 us; at 280 and 320 points even waves lose 7 to 16 %."""
     dbl = elem == 16
     most = 16 if dbl else 32
     if dbl and max(prime_factors(N)) > most:
@@ -114,7 +120,10 @@ def column_radices(N: int, elem: int, B: int) -> Optional[Tuple[Tuple[int, ...],
                     continue
                 lanes = -(-tt * B // WAVE) * WAVE / (tt * B)
                 work = sum(slots(N, r, tt) * tt for r in rads) / N * lanes
-                cost = 0.1 * count + 0.223 * work + 0.464 * max(0, values - (12 if dbl else 20)) / most
+                waves = -(-tt * B // WAVE)
+                uneven = -(-waves // 4) * 4 / waves - 1 if waves > 4 and B * N * elem > UNEVEN_LDS else 0.0
+                cost = (0.1 * count + 0.223 * work + 0.464 * max(0, values - (12 if dbl else 20)) / most
+                        + 0.38 * uneven)
                 key = (round(cost, 6), rads[::-1], tt)
                 if best is None or key < best:
                     best = key
