@@ -337,7 +337,10 @@ template <class C> __device__ __forceinline__ Geo make_geo() {
   if constexpr (C::S > 1) {
     g.outer = wg / C::NWG_INNER;
     g.inner = (wg % C::NWG_INNER) * C::B + (u32)g.b;
-    g.valid = g.inner < C::S && g.outer < C::OUTER;  // (the grid may end in idle workgroups)
+    g.valid = g.inner < C::S;
+    if constexpr (xcdmap_of<C>::value) {
+      if constexpr (C::NWG > C::OUTER * C::NWG_INNER) g.valid = g.valid && g.outer < C::OUTER;  // idle workgroups
+    }
   } else {
     g.outer = wg * C::B + (u32)g.b;
     g.inner = 0;
