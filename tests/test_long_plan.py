@@ -61,3 +61,24 @@ def test_what_does_not_split():
     """Prime factors above 13, short lengths and lengths beyond two tiles stay elsewhere."""
     for n in (17 * 1024, 65537, 2048, 1 << 26):
         assert LG.split_length(n) is None
+
+
+def test_scratch_of_streams_and_captures(monkeypatch):
+    """Two streams never share what lies between the launches, nor do a capture and the
+    launches that follow it; what a plan keeps is bounded."""
+    import threading
+    capturing = set()
+    monkeypatch.setattr(LG, "Buffer", lambda shape, dtype: object())
+    monkeypatch.setattr(LG.rt, "is_capturing", lambda s=None: s in capturing)
+    plan = object.__new__(LG.LongFFT)
+    plan._points, plan._scratch, plan._captured, plan._lock = 8, {}, None, threading.Lock()
+    got = {s: plan._scratch_for(s) for s in range(7)}
+    assert len({id(b) for b in got.values()}) == 7 and len(plan._scratch) == LG.SCRATCH_STREAMS
+    assert plan._scratch_for(6) is got[6] and plan._scratch_for(0) is not got[0]
+    for stream in (6, 99):  # warmed up on this stream, and not
+        plan._captured = None
+        capturing = {stream}
+        taken = plan._scratch_for(stream)
+        assert plan._scratch_for(stream) is taken
+        capturing = set()
+        assert all(plan._scratch_for(s) is not taken for s in range(7)) and plan._scratch_for(stream) is not taken

@@ -27,6 +27,7 @@ from .prime_utils import prime_factors
 MAX_PRIME = 13        # larger prime factors go through Bluestein (fft/ragged.py)
 MAX_RADIX = 32        # complex64 values a thread holds at most (64 registers)
 TILE_MAX = 4096       # longest column or row: 4 of them (32-byte runs) still fit LDS
+SCRATCH_STREAMS = 4   # streams whose buffers a plan keeps
 CHUNK_POINTS = 1 << 23  # points per pair of launches: 64 MiB of scratch, which stays in the 256 MB cache
 
 
@@ -218,20 +219,27 @@ class LongFFT:
         # whole row tiles of the largest chunk (the tile of a smaller one may be narrower)
         self._points = max(c * scratch_points(self.n, k[1].plan.B) for c, k in self.kernels.items())
         self._scratch: Dict[int, Buffer] = {}
+        self._captured: Optional[Buffer] = None
         self._lock = threading.Lock()
 
     def _scratch_for(self, stream: int) -> Buffer:
         """The data between the launches, one buffer per stream: launches on different
-        streams may overlap.  A capture cannot allocate; it takes the first one."""
-        s = self._scratch.get(stream)
-        if s is None:
-            with self._lock:
-                s = self._scratch.get(stream)
-                if s is None:
-                    if self._scratch and (len(self._scratch) >= 4 or rt.is_capturing(stream)):
-                        return next(iter(self._scratch.values()))
-                    s = self._scratch[stream] = Buffer((self._points,), dt.complex64)
-        return s
+        streams may overlap.  The plan keeps those of the last SCRATCH_STREAMS streams; an
+        older one lives on while a bound launch holds it.  A capture cannot allocate: the
+        first takes a buffer that no stream's launches use from then on, and the plan keeps
+        it for the replays (captures of one plan share it: replays must not overlap)."""
+        with self._lock:
+            if rt.is_capturing(stream):
+                if self._captured is None:
+                    if not self._scratch:
+                        rt.require_not_capturing("the first call of a long transform")
+                    self._captured = self._scratch.pop(stream, None) or self._scratch.popitem()[1]
+                return self._captured
+            s = self._scratch.pop(stream, None) or Buffer((self._points,), dt.complex64)
+            self._scratch[stream] = s  # the newest comes last
+            while len(self._scratch) > SCRATCH_STREAMS:
+                del self._scratch[next(iter(self._scratch))]
+            return s
 
     def bind(self, buf):
         """``launch(stream)`` for this buffer; it allocates nothing (safe under graph capture)."""
