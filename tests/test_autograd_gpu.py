@@ -134,3 +134,19 @@ def test_packed_columns_and_their_adjoint(shape, dtype, which):
             continue
         ref = want[name]
         assert float((got.cpu().double() - ref).norm() / ref.norm()) < tol, name
+
+
+def test_nothing_is_kept_without_a_backward_pass(monkeypatch):
+    """Under no_grad a learnable kernel takes the launch that stores no transforms."""
+    from vkdispatch_amd.fft import autograd
+    kept = []
+    forward = autograd._forward
+    monkeypatch.setattr(autograd, "_forward", lambda x, k, plans, keep=False: kept.append(keep) or
+                        forward(x, k, plans, keep))
+    x = torch.randn(2, 64, 48, device="cuda")
+    k = torch.randn(64, 48, device="cuda", requires_grad=True)
+    with torch.no_grad():
+        y0 = _fft_conv()(x, k)
+    y1 = _fft_conv()(x, k)
+    assert kept == [False, True] and not y0.requires_grad and y1.requires_grad
+    assert torch.equal(y0, y1.detach())

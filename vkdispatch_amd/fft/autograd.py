@@ -292,6 +292,9 @@ def fft_convolve2d(x, k):
     global _FN
     if _FN is None:
         _FN = _autograd_function()
+    torch = _torch()
+    if not torch.is_grad_enabled() and isinstance(k, torch.Tensor):
+        k = k.detach()  # no backward pass: nothing is kept for the gradient of k
     return _FN.apply(x, k)
 
 
