@@ -5,6 +5,7 @@ import pytest
 
 import vkdispatch_amd as vd
 from vkdispatch_amd.fft import planner as P
+from vkdispatch_amd.fft.shader_factories import make_convolution_shader, make_fft_shader
 
 LENGTHS = [33, 34, 40, 60, 96, 100, 162, 243, 480, 600, 961, 1000, 1024, 1155, 2048, 2160, 4096, 8192, 9282, 10000,
            13122, 14406, 16384]
@@ -64,3 +65,25 @@ def test_transposed_layout_is_what_it_was(shape, axis, size):
     t = vd.fft.make_transpose_shader(shape, axis)
     assert list(k.plan.radices) == P.radix_plan(shape[axis])[0] and k.plan.TT == P.radix_plan(shape[axis])[1]
     assert (k.plan.B, k.plan.NWG, k.plan.LPW) == (t.plan.B, t.plan.NWG, 0)
+
+
+@pytest.mark.parametrize("shape,real,conv,want", [
+    ((1, 640, 320), "float", True, (1, 2)), ((1, 640, 320), "float", False, (1, 2)),    # few workgroups
+    ((26, 500, 320), "float", True, (2, 3)), ((65, 200, 320), "float", True, (1, 3)),
+    ((26, 500, 320), "float", False, None), ((32, 400, 320), "float", True, None),      # measured slower
+    ((20, 640, 320), "float", True, None),                                              # 8 waves a workgroup
+    ((26, 500, 257), "float", True, None), ((64, 512, 1), "float", True, None),         # part tiles, rows
+    ((40, 160, 320), "double", False, (1, 3)), ((40, 160, 320), "double", True, None)])
+def test_waves_to_schedule_for(shape, real, conv, want):
+    """The bound holds the workgroup's own waves, and what it gives the compiler spills nothing."""
+    plan = P.make_plan(P.AxisGeometry.of(shape, 1), real, kind="conv" if conv else "fft")
+    got = P.wave_bounds(plan, conv)
+    assert got == want
+    if got is None:
+        return
+    assert got[0] <= got[1] and 4 * P.WAVE * got[0] >= plan.BLOCK
+    c = vd.complex64 if real == "float" else vd.complex128
+    k = make_convolution_shader(shape, None, 1, 1, kernel_inner_only=True) if conv else \
+        make_fft_shader(shape, 1, input_type=c, output_type=c, compute_type=c)
+    assert f"amdgpu_waves_per_eu({got[0]}, {got[1]})" in k.source
+    assert k.code_object_info()["private_bytes"] == 0

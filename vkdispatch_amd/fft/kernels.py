@@ -170,10 +170,13 @@ def source_symbol(source: str) -> str:
     return m.group(1)
 
 
-def translation_unit(cfg: str, functors: Sequence[str], body: str, block: int, symbol: str = "vkx_main") -> str:
+def translation_unit(cfg: str, functors: Sequence[str], body: str, block: int, symbol: str = "vkx_main",
+                     waves: Optional[Tuple[int, int]] = None) -> str:
+    """``waves``: least and most waves per SIMD that the compiler is to schedule for."""
     parts = ['#include "vkx_fft.h"', "", cfg, ""]
     parts += list(functors)
-    parts += ["", f'extern "C" __global__ void __launch_bounds__({block}) {symbol}(vkx::KParams prm) {{',
+    occ = f" __attribute__((amdgpu_waves_per_eu({waves[0]}, {waves[1]})))" if waves else ""
+    parts += ["", f'extern "C" __global__ void __launch_bounds__({block}){occ} {symbol}(vkx::KParams prm) {{',
               f"  {body}", "}", ""]
     return "\n".join(parts)
 

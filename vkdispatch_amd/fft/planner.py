@@ -413,6 +413,34 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
                       NWG_INNER=nwg_inner, TWREG=twreg, LPW=lpw, CPAD=cpad)
 
 
+def wave_bounds(plan: KernelPlan, conv: bool) -> Optional[Tuple[int, int]]:
+    """Least and most waves per SIMD to schedule a strided kernel for, or None: the
+    compiler's own choice.  Where every tile is full (no guard keeps the loads together)
+    and a thread holds many values, the compiler goes for four waves and up by putting
+    each read of K and of a twiddle next to its use, up to 60 of them one after another,
+    each waited for.  A launch that does not fill the chip has nothing to gain from more
+    waves (1 x 640 x 320: convolved 13.7 -> 9.3 us, transformed 8.1 -> 6.3; 35 lengths of
+    36 to 1024 convolved 14 % faster, the worst 2 % slower).  Others take three waves
+    where they measured faster: convolutions with 24 values and up (26 x 500 x 320
+    42.9 -> 30.7, 136 x 96 x 320 23.1 -> 15.8; with 20 and 21 values 300 to 400 points lose
+    20 %, but 65 x 200 x 320, whose LDS allows six workgroups on a CU, 33.6 -> 19.3;
+    workgroups of 8 waves have a second one on the CU only with four waves: 28.7 -> 31.3),
+    complex128 transforms with 16 (40 x 160 x 320 14.4 -> 12.3, none slower than 2 %);
+    complex64 transforms lose 4 %."""
+    dbl = plan.real == "double"
+    if not plan.COLFAST or plan.S % plan.B or plan.TT == 1 or plan.BLOCK > 512 or plan.VMAX < (16 if dbl else 20):
+        return None
+    least = -(-plan.BLOCK // (4 * WAVE))  # a workgroup's own
+    if dbl:
+        return None if conv else (least, 3)
+    if plan.NWG < 256:
+        return least, 2
+    lds = plan.LDS_ELEMS * 8
+    if conv and plan.BLOCK < 512 and (plan.VMAX >= 24 or (lds < 32 * 1024 and plan.BLOCK > WAVE)):
+        return least, 3
+    return None
+
+
 def whole_xcds(plan: KernelPlan) -> KernelPlan:
     """The plan with a grid of 8k workgroups (the last ones idle), as the XCD order needs."""
     return dataclasses.replace(plan, NWG=-(-plan.NWG // 8) * 8) if plan.NWG >= 16 else plan

@@ -13,7 +13,7 @@ from typing import Optional, Tuple
 from .. import dtypes as dt
 from . import hooks
 from .kernels import CompiledKernel, cfg_struct, kernel_symbol, translation_unit
-from .planner import AxisGeometry, KernelPlan, make_plan, transposed_size, whole_xcds
+from .planner import AxisGeometry, KernelPlan, make_plan, transposed_size, wave_bounds, whole_xcds
 from .precision import kernel_real_type
 
 
@@ -113,7 +113,8 @@ def make_fft_shader(buffer_shape: Tuple, axis: int = None, inverse: bool = False
     kind = ("irfft" if inverse else "rfft") if r2c else "fft"
     tag = ("inv" if inverse else "fwd") + ("_hook" if (input_map or output_map) else "")
     src = translation_unit(cfg, functors, "vkx::fft_body<Cfg, HookIn, HookOut>(prm);", plan.BLOCK,
-                           kernel_symbol(kind, plan, tag))
+                           kernel_symbol(kind, plan, tag),
+                           None if input_map or output_map else wave_bounds(plan, False))
     name = f"fft_shader_{tuple(buffer_shape)}_{axis}_{inverse}_{normalize_inverse}_{r2c}"
     return CompiledKernel(src, plan, args, list(plan.radices), None, name=name)
 
@@ -236,8 +237,9 @@ def make_convolution_shader(buffer_shape: Tuple, kernel_map=None, kernel_num: in
         functors.append(f"using HookKernel = vkx::DefaultKernel<{k_args[0].slot}, {kernel_type.child_type.cpp}>;")
     tag = ("inner" if kernel_inner_only else "") + ("_t" if transposed_kernel else "") + \
         ("_hook" if (input_map or output_map or kernel_map) else "") + (f"_k{kernel_num}" if kernel_num > 1 else "")
+    plain = not (input_map or output_map or kernel_map or transposed_kernel) and kernel_num == 1
     src = translation_unit(cfg, functors, "vkx::conv_body<Cfg, HookIn, HookKernel, HookOut>(prm);", plan.BLOCK,
-                           kernel_symbol("conv", plan, tag))
+                           kernel_symbol("conv", plan, tag), wave_bounds(plan, True) if plain else None)
     return CompiledKernel(src, plan, args, list(plan.radices), list(reversed(plan.radices)),
                           name=f"convolution_shader_{tuple(buffer_shape)}_{axis}")
 
