@@ -73,7 +73,8 @@ def test_transposed_layout_is_what_it_was(shape, axis, size):
     ((26, 500, 320), "float", False, None), ((32, 400, 320), "float", True, None),      # measured slower
     ((20, 640, 320), "float", True, None),                                              # 8 waves a workgroup
     ((26, 500, 257), "float", True, None), ((64, 512, 1), "float", True, None),         # part tiles, rows
-    ((40, 160, 320), "double", False, (1, 3)), ((40, 160, 320), "double", True, None)])
+    ((40, 160, 320), "double", False, (1, 3)), ((72, 90, 320), "double", False, (1, 3)),
+    ((40, 160, 320), "double", True, None)])
 def test_waves_to_schedule_for(shape, real, conv, want):
     """The bound holds the workgroup's own waves, and what it gives the compiler spills nothing."""
     plan = P.make_plan(P.AxisGeometry.of(shape, 1), real, kind="conv" if conv else "fft")

@@ -70,7 +70,7 @@ def test_signal_range_with_idle_lanes():
     assert_close(buf.read(0), O.fft_axis(part, 1))
 
 
-@pytest.mark.parametrize("shape", [(1, 640, 32), (3, 500, 16), (70, 96, 64), (65, 200, 64), (26, 540, 160)], ids=str)
+@pytest.mark.parametrize("shape", [(1, 640, 32), (3, 500, 16), (70, 96, 64), (65, 200, 64), (26, 540, 160), (70, 90, 32)], ids=str)
 def test_kernels_scheduled_for_fewer_waves(shape):
     """Full tiles of many values a thread: launches that leave CUs idle, and others."""
     test_convolution(shape, "inner")

@@ -425,10 +425,10 @@ def wave_bounds(plan: KernelPlan, conv: bool) -> Optional[Tuple[int, int]]:
     42.9 -> 30.7, 136 x 96 x 320 23.1 -> 15.8; with 20 and 21 values 300 to 400 points lose
     20 %, but 65 x 200 x 320, whose LDS allows six workgroups on a CU, 33.6 -> 19.3;
     workgroups of 8 waves have a second one on the CU only with four waves: 28.7 -> 31.3),
-    complex128 transforms with 16 (40 x 160 x 320 14.4 -> 12.3, none slower than 2 %);
+    complex128 transforms with 15 and 16 (40 x 160 x 320 14.4 -> 12.3, none slower than 2 %);
     complex64 transforms lose 4 %."""
     dbl = plan.real == "double"
-    if not plan.COLFAST or plan.S % plan.B or plan.TT == 1 or plan.BLOCK > 512 or plan.VMAX < (16 if dbl else 20):
+    if not plan.COLFAST or plan.S % plan.B or plan.TT == 1 or plan.BLOCK > 512 or plan.VMAX < (15 if dbl else 20):
         return None
     least = -(-plan.BLOCK // (4 * WAVE))  # a workgroup's own
     if dbl:
