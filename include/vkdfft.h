@@ -62,6 +62,10 @@ int vkx_device_props_get(int device, vkx_device_props* out);
 /* ---- memory ---------------------------------------------------------------- */
 /* replaces native.buffer_create / buffer_destroy (vkdispatch/base/buffer.py:101-128,140-147) */
 int vkx_malloc(uint64_t* dptr, size_t bytes);
+/* the same while a stream of this thread is being captured into a graph: the allocation is
+ * made at once and is no part of the capture (vkdispatch allocates before recording,
+ * vkdispatch/execution_pipeline/cuda_graph_capture.py:22-52) */
+int vkx_malloc_capturing(uint64_t* dptr, size_t bytes);
 int vkx_free(uint64_t dptr);
 /* replace native.buffer_write_staging + buffer_write and buffer_read +
  * buffer_read_staging (vkdispatch/base/buffer.py:154-258) */

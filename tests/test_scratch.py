@@ -1,0 +1,107 @@
+"""Who shares what lies between the launches of one call: kernels and buffers that only note
+what is done with them, on the CPU."""
+import threading
+
+import pytest
+
+from vkdispatch_amd import graph as G
+from vkdispatch_amd import runtime as rt
+from vkdispatch_amd.fft import functions as F
+from vkdispatch_amd.fft import long as LG
+
+
+class _Kernel:
+    def __init__(self, log, name):
+        self.log, self.name = log, name
+
+    def handle(self):
+        return 1
+
+    def launch_raw(self, ptrs, consts=b"", stream=None):
+        self.log.append((self.name, stream, tuple(ptrs)))
+
+
+class _Data:
+    def __init__(self, ptr, size=1 << 20):
+        self.ptr, self.size = ptr, size
+
+
+@pytest.fixture
+def device(monkeypatch):
+    """The allocator's addresses, the current stream and what is being captured, as the
+    test sets them; freed addresses are listed."""
+    class Device:
+        stream, capturing, freed, next_ptr = 1, {}, [], 1 << 20
+    dev = Device()
+    dev.capturing, dev.freed = {}, []
+
+    def malloc(nbytes):
+        dev.next_ptr += 1 << 20
+        return dev.next_ptr
+    monkeypatch.setattr(rt, "malloc", malloc)
+    monkeypatch.setattr(rt, "free", dev.freed.append)
+    monkeypatch.setattr(rt, "synchronize", lambda stream=None: None)
+    monkeypatch.setattr(rt, "current_stream", lambda: dev.stream)
+    monkeypatch.setattr(rt, "is_capturing", lambda s=None: (dev.stream if s is None else s) in dev.capturing)
+    return dev
+
+
+def _long_plan(points=64):
+    """A LongFFT of 3 transforms in two chunks, its kernels noting their launches."""
+    log = []
+    plan = object.__new__(LG.LongFFT)
+    cols, rows = _Kernel(log, "cols"), _Kernel(log, "rows")
+    plan.n, plan.count, plan.chunks = 16, 3, [(0, 2), (2, 1)]
+    plan.kernels = {1: (cols, rows), 2: (cols, rows)}
+    plan.tables = (_Data(5), _Data(6))
+    plan._points, plan._scratch, plan._captured, plan._lock = points, {}, None, threading.Lock()
+    return plan, log
+
+
+def _between(log):
+    """(stream, scratch address) of every pair of launches, which must be the same in both."""
+    out = []
+    for (a, s, p), (b, t, q) in zip(log[::2], log[1::2]):
+        assert (a, b) == ("cols", "rows") and s == t and p[0] == q[1]
+        out.append((s, p[0]))
+    return out
+
+
+def _call(plan, monkeypatch, buf, graph=None):
+    """fft() of a long length as functions.py routes it."""
+    monkeypatch.setattr(F, "_uniform_plan", lambda *a: plan)
+    from vkdispatch_amd import dtypes as dt
+    assert F._large_or_prime_fallback((buf,), (3, 1 << 20), None, False, True, False, None, None, dt.complex64,
+                                      dt.complex64, None, graph)
+
+
+def test_recorded_long_transforms_share_nothing_with_calls(device, monkeypatch):
+    """Recorded on one stream and submitted on another beside calls on the first; two graphs
+    recorded on one stream and submitted on two; the launches of one graph share."""
+    plan, log = _long_plan()
+    graphs = [G.CommandGraph(), G.CommandGraph()]
+    for g in graphs:
+        for b in (100, 200):
+            _call(plan, monkeypatch, _Data(b), g)
+    assert not log
+    for g, s in zip(graphs, (2, 3)):
+        g._replay(s)
+    _call(plan, monkeypatch, _Data(300))
+    used = {}
+    for s, y in _between(log):
+        used.setdefault(s, set()).add(y)
+    assert sorted(used) == [1, 2, 3] and all(len(v) == 1 for v in used.values())
+    assert len(set.union(*used.values())) == 3
+    assert not device.freed
+    y2 = used[2]
+    graphs[0].reset()
+    assert set(device.freed) == y2
+
+
+def test_a_bound_long_transform_has_its_own_scratch(device):
+    plan, log = _long_plan()
+    a, b = plan.bind(_Data(100)), plan.bind(_Data(200))
+    plan(_Data(300))
+    a(1)
+    b(1)
+    assert len({y for _, y in _between(log)}) == 3

@@ -296,6 +296,17 @@ int vkx_malloc(uint64_t* dptr, size_t bytes) {
   return 0;
 }
 
+int vkx_malloc_capturing(uint64_t* dptr, size_t bytes) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  VKX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  void* p = nullptr;
+  const hipError_t made = hipMalloc(&p, bytes ? bytes : 1);
+  VKX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  VKX_HIP(made);
+  *dptr = reinterpret_cast<uint64_t>(p);
+  return 0;
+}
+
 int vkx_free(uint64_t dptr) {
   if (dptr) VKX_HIP(hipFree(reinterpret_cast<void*>(dptr)));
   return 0;

@@ -173,10 +173,11 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
     if (geom.S != 1 or r2c or input_map is not None or output_map is not None or signal_range is not None
             or out_t is not dt.complex64 or comp_t not in (dt.complex64, dt.complex32)):
         return False
+    from .long import LongFFT
     plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize))
     buf = buffers[0]
-    if graph is not None:
-        graph.record_callable(plan.bind(buf))
+    if graph is not None and not graph.submit_on_record:
+        graph.record_callable(plan.bind(buf, graph=graph) if isinstance(plan, LongFFT) else plan.bind(buf))
     else:
         plan(buf)
     return True

@@ -223,9 +223,9 @@ class LongFFT:
         self._lock = threading.Lock()
 
     def _scratch_for(self, stream: int) -> Buffer:
-        """The data between the launches, one buffer per stream: launches on different
-        streams may overlap.  The plan keeps those of the last SCRATCH_STREAMS streams; an
-        older one lives on while a bound launch holds it.  A capture cannot allocate: the
+        """The data between the launches of a call, one buffer per stream: calls on different
+        streams may overlap.  The plan keeps those of the last SCRATCH_STREAMS streams (a
+        further one frees the oldest, which waits for the GPU).  A capture cannot allocate: the
         first takes a buffer that no stream's launches use from then on, and the plan keeps
         it for the replays (captures of one plan share it: replays must not overlap)."""
         with self._lock:
@@ -241,18 +241,30 @@ class LongFFT:
                 del self._scratch[next(iter(self._scratch))]
             return s
 
-    def bind(self, buf):
-        """``launch(stream)`` for this buffer; it allocates nothing (safe under graph capture)."""
+    def _new_scratch(self) -> Buffer:
+        with rt.allocating_in_capture():  # launches may be recorded while a caller captures
+            return Buffer((self._points,), dt.complex64)
+
+    def _launches(self, buf, y) -> list:
+        """(kernel, pointers) of every launch, through scratch ``y``."""
         if buf.size < self.n * self.count:
             raise ValueError(f"buffer of {buf.size} elements, the batch needs {self.n * self.count}")
-        y = self._scratch_for(rt.current_stream())
         a, r = self.tables
         calls = []
         for first, c in self.chunks:
             cols, rows = self.kernels[c]
-            cols.handle(), rows.handle()
             x = int(buf.ptr) + 8 * self.n * first
             calls += [(cols, [y.ptr, x, a.ptr, r.ptr]), (rows, [x, y.ptr])]
+        return calls
+
+    def bind(self, buf, graph=None):
+        """``launch(stream)`` for this buffer; it allocates nothing (safe under graph capture)
+        and has scratch of its own, or that of the CommandGraph it is recorded into: it may
+        run on any stream, beside calls of this plan."""
+        for k in {k for pair in self.kernels.values() for k in pair}:
+            k.handle()
+        y = self._new_scratch() if graph is None else graph.scratch(8 * self._points)
+        calls = self._launches(buf, y)
         keep = (buf, y, self)
 
         def launch(stream=None):
@@ -262,7 +274,10 @@ class LongFFT:
         return launch
 
     def __call__(self, buf) -> None:
-        self.bind(buf)(rt.current_stream())
+        stream = rt.current_stream()
+        y = self._scratch_for(stream)
+        for k, ptrs in self._launches(buf, y):
+            k.launch_raw(ptrs, b"", stream)
 
 
 def clear() -> None:

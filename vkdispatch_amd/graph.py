@@ -24,6 +24,7 @@ class CommandGraph:
         self.submit_on_record = submit_on_record
         # (kernel or launcher, device pointers, packed constants, objects kept alive)
         self._records: List[Tuple[object, Optional[List[int]], Optional[bytes], tuple]] = []
+        self._scratch: List[object] = []
         self._exec: Optional[int] = None
         self._exec_stream: Optional[int] = None
 
@@ -47,6 +48,17 @@ class CommandGraph:
             return
         self._records.append((fn, None, None, ()))
         self._drop_exec()
+
+    def scratch(self, nbytes: int):
+        """A buffer of at least ``nbytes`` for what recorded launches hand to each other.  The
+        launches of a graph run one after another, so they share it; nothing else uses it."""
+        for b in self._scratch:
+            if b.mem_size >= nbytes:
+                return b
+        from .buffer import Buffer
+        with rt.allocating_in_capture():  # launches may be recorded while a caller captures
+            self._scratch.append(Buffer((-(-int(nbytes) // 8),)))
+        return self._scratch[-1]
 
     def __len__(self):
         return len(self._records)
@@ -103,6 +115,7 @@ class CommandGraph:
     def reset(self) -> None:
         self._drop_exec()
         self._records = []
+        self._scratch = []
 
     def destroy(self) -> None:
         self.reset()

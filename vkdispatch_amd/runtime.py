@@ -7,6 +7,7 @@ missing.  There is no CPU fallback anywhere on the product path.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -65,6 +66,7 @@ _SIGS = {
     "vkx_device_count": ([ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
     "vkx_device_props_get": ([ctypes.c_int, ctypes.POINTER(DeviceProps)], ctypes.c_int),
     "vkx_malloc": ([_PU64, ctypes.c_size_t], ctypes.c_int),
+    "vkx_malloc_capturing": ([_PU64, ctypes.c_size_t], ctypes.c_int),
     "vkx_free": ([_U64], ctypes.c_int),
     "vkx_memcpy_htod": ([_U64, ctypes.c_void_p, ctypes.c_size_t, _U64], ctypes.c_int),
     "vkx_memcpy_dtoh": ([ctypes.c_void_p, _U64, ctypes.c_size_t, _U64], ctypes.c_int),
@@ -171,6 +173,7 @@ def check(rc: int, what: str = "") -> None:
 # ---------------------------------------------------------------------------
 class _State(threading.local):
     stream_override = None
+    allocating_in_capture = False
 
 
 _state = _State()
@@ -316,6 +319,17 @@ def is_capturing(stream=None) -> bool:
     return c.value != 0
 
 
+@contextlib.contextmanager
+def allocating_in_capture():
+    """Allocations of this thread are made although a stream is being captured: memory that
+    the captured launches use and that needs no initialisation."""
+    prev, _state.allocating_in_capture = _state.allocating_in_capture, True
+    try:
+        yield
+    finally:
+        _state.allocating_in_capture = prev
+
+
 def require_not_capturing(what: str) -> None:
     """Raise if the current stream is capturing: ``what`` allocates or initialises device
     memory, which a graph capture must not record."""
@@ -337,8 +351,11 @@ def synchronize(stream=None) -> None:
 # ---------------------------------------------------------------------------
 def malloc(nbytes: int) -> int:
     ensure_device()
-    require_not_capturing("a device allocation")
     p = ctypes.c_uint64(0)
+    if _state.allocating_in_capture:
+        check(lib().vkx_malloc_capturing(ctypes.byref(p), max(1, int(nbytes))), "vkx_malloc_capturing")
+        return p.value
+    require_not_capturing("a device allocation")
     check(lib().vkx_malloc(ctypes.byref(p), max(1, int(nbytes))), "vkx_malloc")
     return p.value
 
