@@ -204,6 +204,9 @@ int vkx_graph_begin(uint64_t stream);
  * (vkdispatch/execution_pipeline/cuda_graph_capture.py:22-52): plans refuse to allocate
  * or initialise device memory while their stream is capturing. */
 int vkx_stream_is_capturing(uint64_t stream, int* capturing);
+/* *id = a number that tells captures apart (the same on every stream that takes part in
+ * one), 0 when `stream` is not being captured. */
+int vkx_stream_capture_id(uint64_t stream, uint64_t* id);
 int vkx_graph_end(uint64_t stream, uint64_t* graph_exec);
 int vkx_graph_launch(uint64_t graph_exec, uint64_t stream);
 int vkx_graph_destroy(uint64_t graph_exec);

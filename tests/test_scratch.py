@@ -43,6 +43,7 @@ def device(monkeypatch):
     monkeypatch.setattr(rt, "synchronize", lambda stream=None: None)
     monkeypatch.setattr(rt, "current_stream", lambda: dev.stream)
     monkeypatch.setattr(rt, "is_capturing", lambda s=None: (dev.stream if s is None else s) in dev.capturing)
+    monkeypatch.setattr(rt, "capture_id", lambda s: dev.capturing.get(s, 0), raising=False)
     return dev
 
 
@@ -105,3 +106,29 @@ def test_a_bound_long_transform_has_its_own_scratch(device):
     a(1)
     b(1)
     assert len({y for _, y in _between(log)}) == 3
+
+
+def test_captures_share_nothing(device):
+    """With bound launches, calls on any stream, other captures and their own branches."""
+    plan, log = _long_plan()
+
+    def used(launch, *a):
+        del log[:]
+        launch(*a)
+        (y,) = {y for _, y in _between(log)}
+        return y
+    bound = plan.bind(_Data(100))
+    outside = {used(bound, 7), used(plan, _Data(200))}
+    device.capturing = {1: 11, 2: 11}   # one capture with two branches
+    first = [used(plan, _Data(300)) for device.stream in (1, 2)]
+    assert [used(plan, _Data(300)) for device.stream in (1, 2)] == first
+    device.capturing = {1: 12}          # another on a stream that had one before
+    device.stream = 1
+    first.append(used(plan, _Data(300)))
+    device.capturing = {}
+    outside |= {used(plan, _Data(400)) for device.stream in (1, 2, 3, 4)} | {used(bound, 7)}
+    assert len(set(first)) == 3 and not outside & set(first)
+    for device.capturing in [{1: n} for n in range(20, 60)]:
+        device.stream = 1
+        used(plan, _Data(300))
+    assert len(plan._captured) == LG.SCRATCH_CAPTURES and not set(device.freed) & set(first)

@@ -633,6 +633,15 @@ int vkx_stream_is_capturing(uint64_t stream, int* capturing) {
   return 0;
 }
 
+int vkx_stream_capture_id(uint64_t stream, uint64_t* id) {
+  *id = 0;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  unsigned long long n = 0;
+  VKX_HIP(hipStreamGetCaptureInfo(S(stream), &st, &n));
+  if (st == hipStreamCaptureStatusActive) *id = n;
+  return 0;
+}
+
 int vkx_graph_begin(uint64_t stream) {
   VKX_HIP(hipStreamBeginCapture(S(stream), hipStreamCaptureModeThreadLocal));
   return 0;

@@ -28,6 +28,8 @@ MAX_PRIME = 13        # larger prime factors go through Bluestein (fft/ragged.py
 MAX_RADIX = 32        # complex64 values a thread holds at most (64 registers)
 TILE_MAX = 4096       # longest column or row: 4 of them (32-byte runs) still fit LDS
 SCRATCH_STREAMS = 4   # streams whose buffers a plan keeps
+SCRATCH_CAPTURES = 16  # captures with a buffer of their own; the next one takes the oldest's, and replays
+#                        of those two must not overlap
 CHUNK_POINTS = 1 << 23  # points per pair of launches: 64 MiB of scratch, which stays in the 256 MB cache
 
 
@@ -219,27 +221,30 @@ class LongFFT:
         # whole row tiles of the largest chunk (the tile of a smaller one may be narrower)
         self._points = max(c * scratch_points(self.n, k[1].plan.B) for c, k in self.kernels.items())
         self._scratch: Dict[int, Buffer] = {}
-        self._captured: Optional[Buffer] = None
+        self._captured: Dict[Tuple[int, int], Buffer] = {}
         self._lock = threading.Lock()
 
     def _scratch_for(self, stream: int) -> Buffer:
         """The data between the launches of a call, one buffer per stream: calls on different
         streams may overlap.  The plan keeps those of the last SCRATCH_STREAMS streams (a
-        further one frees the oldest, which waits for the GPU).  A capture cannot allocate: the
-        first takes a buffer that no stream's launches use from then on, and the plan keeps
-        it for the replays (captures of one plan share it: replays must not overlap)."""
+        further one frees the oldest, which waits for the GPU).  A call inside a capture of the
+        caller's takes a buffer that the plan keeps for this capture: its replays may run at
+        any time and on any stream."""
         with self._lock:
             if rt.is_capturing(stream):
-                if self._captured is None:
-                    if not self._scratch:
-                        rt.require_not_capturing("the first call of a long transform")
-                    self._captured = self._scratch.pop(stream, None) or self._scratch.popitem()[1]
-                return self._captured
-            s = self._scratch.pop(stream, None) or Buffer((self._points,), dt.complex64)
+                return self._scratch_of_capture(stream)
+            s = self._scratch.pop(stream, None) or self._new_scratch()
             self._scratch[stream] = s  # the newest comes last
             while len(self._scratch) > SCRATCH_STREAMS:
                 del self._scratch[next(iter(self._scratch))]
             return s
+
+    def _scratch_of_capture(self, stream: int) -> Buffer:
+        kept = self._captured = self._captured or {}
+        key = (rt.capture_id(stream), stream)  # the branches of one capture may overlap, too
+        if key not in kept:
+            kept[key] = self._new_scratch() if len(kept) < SCRATCH_CAPTURES else kept.pop(next(iter(kept)))
+        return kept[key]
 
     def _new_scratch(self) -> Buffer:
         with rt.allocating_in_capture():  # launches may be recorded while a caller captures

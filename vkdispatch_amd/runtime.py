@@ -110,6 +110,7 @@ _SIGS = {
     "vkx_bluestein_b": ([_U64, ctypes.c_int, ctypes.c_int, _U64], ctypes.c_int),
     "vkx_graph_begin": ([_U64], ctypes.c_int),
     "vkx_stream_is_capturing": ([_U64, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
+    "vkx_stream_capture_id": ([_U64, _PU64], ctypes.c_int),
     "vkx_graph_end": ([_U64, _PU64], ctypes.c_int),
     "vkx_graph_launch": ([_U64, _U64], ctypes.c_int),
     "vkx_graph_destroy": ([_U64], ctypes.c_int),
@@ -317,6 +318,15 @@ def is_capturing(stream=None) -> bool:
     check(lib().vkx_stream_is_capturing(current_stream() if stream is None else int(stream), ctypes.byref(c)),
           "vkx_stream_is_capturing")
     return c.value != 0
+
+
+def capture_id(stream: int) -> int:
+    """A number that tells the captures under way on ``stream`` apart (0: none)."""
+    if not device_initialised():
+        return 0
+    n = ctypes.c_uint64(0)
+    check(lib().vkx_stream_capture_id(int(stream), ctypes.byref(n)), "vkx_stream_capture_id")
+    return n.value
 
 
 @contextlib.contextmanager
