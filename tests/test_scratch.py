@@ -132,3 +132,37 @@ def test_captures_share_nothing(device):
         device.stream = 1
         used(plan, _Data(300))
     assert len(plan._captured) == LG.SCRATCH_CAPTURES and not set(device.freed) & set(first)
+
+
+def test_two_threads_on_one_stream_take_turns(device):
+    """The second thread calls while the first is between its launches; on the stream of each
+    thread (one handle, hipStreamPerThread) they have different scratch."""
+    for stream, apart in ((1, False), (2, True)):
+        device.stream = stream
+        plan, log = _long_plan()
+        inside, other = threading.Event(), threading.Event()
+
+        class Slow(_Kernel):
+            def launch_raw(self, ptrs, consts=b"", stream=None):
+                super().launch_raw(ptrs, consts, stream)
+                if not inside.is_set():
+                    inside.set()
+                    other.wait(0.3)    # as long as the other thread would need
+        rows = plan.kernels[1][1]
+        plan.kernels = {c: (Slow(log, "cols"), rows) for c in (1, 2)}
+
+        def second():
+            inside.wait()
+            plan(_Data(1 << 30))
+            other.set()
+        t = threading.Thread(target=second)
+        t.start()
+        plan(_Data(1 << 25))
+        t.join()
+        if not apart:
+            _between(log)              # whole pairs,
+            x = [p[1] if k == "cols" else p[0] for k, _, p in log]
+            assert len(log) == 8 and [v < 1 << 29 for v in x] in ([True] * 4 + [False] * 4, [False] * 4 + [True] * 4)
+        else:
+            y = {(p[1] if k == "cols" else p[0]) < 1 << 29: p[0] if k == "cols" else p[1] for k, _, p in log}
+            assert len(set(y.values())) == 2

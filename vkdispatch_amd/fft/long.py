@@ -203,6 +203,20 @@ def _twiddles(n: int, radix: int) -> Tuple[Buffer, Buffer]:
     return out[0], out[1]
 
 
+_order = [threading.RLock() for _ in range(16)]
+_PER_THREAD_STREAM = 2  # hipStreamPerThread: one handle for a stream of each thread
+
+
+def _stream_key(stream: int):
+    return (stream, threading.get_ident()) if stream == _PER_THREAD_STREAM else stream
+
+
+def launch_order(stream: int):
+    """Held while a call enqueues its launches on ``stream``: they use the stream's scratch,
+    and another thread's must not come in between."""
+    return _order[hash(_stream_key(stream)) % len(_order)]
+
+
 class LongFFT:
     """``count`` packed transforms of one length that split_length() cuts, in place in a
     complex64 buffer.  A batch of more than CHUNK_POINTS points runs in chunks of whole
@@ -233,15 +247,16 @@ class LongFFT:
         with self._lock:
             if rt.is_capturing(stream):
                 return self._scratch_of_capture(stream)
-            s = self._scratch.pop(stream, None) or self._new_scratch()
-            self._scratch[stream] = s  # the newest comes last
+            key = _stream_key(stream)
+            s = self._scratch.pop(key, None) or self._new_scratch()
+            self._scratch[key] = s  # the newest comes last
             while len(self._scratch) > SCRATCH_STREAMS:
                 del self._scratch[next(iter(self._scratch))]
             return s
 
     def _scratch_of_capture(self, stream: int) -> Buffer:
         kept = self._captured = self._captured or {}
-        key = (rt.capture_id(stream), stream)  # the branches of one capture may overlap, too
+        key = (rt.capture_id(stream), _stream_key(stream))  # the branches of one capture may overlap, too
         if key not in kept:
             kept[key] = self._new_scratch() if len(kept) < SCRATCH_CAPTURES else kept.pop(next(iter(kept)))
         return kept[key]
@@ -280,9 +295,10 @@ class LongFFT:
 
     def __call__(self, buf) -> None:
         stream = rt.current_stream()
-        y = self._scratch_for(stream)
-        for k, ptrs in self._launches(buf, y):
-            k.launch_raw(ptrs, b"", stream)
+        with launch_order(stream):
+            y = self._scratch_for(stream)
+            for k, ptrs in self._launches(buf, y):
+                k.launch_raw(ptrs, b"", stream)
 
 
 def clear() -> None:
