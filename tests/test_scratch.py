@@ -166,3 +166,24 @@ def test_two_threads_on_one_stream_take_turns(device):
         else:
             y = {(p[1] if k == "cols" else p[0]) < 1 << 29: p[0] if k == "cols" else p[1] for k, _, p in log}
             assert len(set(y.values())) == 2
+
+
+def test_plans_on_one_stream_share_a_buffer(device, monkeypatch):
+    """What calls keep grows with the largest plan and the streams, not with the plans."""
+    from vkdispatch_amd.fft import scratch
+    monkeypatch.setattr(scratch, "_streams", {})
+    plans = []
+    for points in (64, 32, 128, 64):
+        plan, log = _long_plan(points)
+        plan._init_scratch()
+        plans.append((plan, log))
+        plan(_Data(100))
+    got = [_between(log)[0][1] for _, log in plans]
+    assert got[0] == got[1] and got[2] == got[3] != got[0]  # the third needs more
+    assert device.freed == [got[0]] and len(scratch._streams) == 1
+    for device.stream in range(20):
+        plans[0][0](_Data(100))
+    assert len(scratch._streams) == scratch.SCRATCH_STREAMS
+    monkeypatch.setattr(scratch, "_pinned", [])
+    scratch.clear()
+    assert not scratch._streams and len(device.freed) == 21

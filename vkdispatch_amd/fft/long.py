@@ -12,7 +12,6 @@ from __future__ import annotations
 
 import dataclasses
 import math
-import threading
 from functools import lru_cache
 from typing import Dict, List, Optional, Tuple
 
@@ -23,13 +22,11 @@ from .hooks import Arg
 from .kernels import CompiledKernel, check_no_spill, kernel_symbol, translation_unit
 from .planner import LDS_BYTES_MAX, MAX_THREADS, KernelPlan, groupings, pass_list, slots
 from .prime_utils import prime_factors
+from .scratch import SCRATCH_CAPTURES, SCRATCH_STREAMS, StreamScratch, launch_order  # noqa: F401
 
 MAX_PRIME = 13        # larger prime factors go through Bluestein (fft/ragged.py)
 MAX_RADIX = 32        # complex64 values a thread holds at most (64 registers)
 TILE_MAX = 4096       # longest column or row: 4 of them (32-byte runs) still fit LDS
-SCRATCH_STREAMS = 4   # streams whose buffers a plan keeps
-SCRATCH_CAPTURES = 16  # captures with a buffer of their own; the next one takes the oldest's, and replays
-#                        of those two must not overlap
 CHUNK_POINTS = 1 << 23  # points per pair of launches: 64 MiB of scratch, which stays in the 256 MB cache
 
 
@@ -203,21 +200,7 @@ def _twiddles(n: int, radix: int) -> Tuple[Buffer, Buffer]:
     return out[0], out[1]
 
 
-_order = [threading.RLock() for _ in range(16)]
-_PER_THREAD_STREAM = 2  # hipStreamPerThread: one handle for a stream of each thread
-
-
-def _stream_key(stream: int):
-    return (stream, threading.get_ident()) if stream == _PER_THREAD_STREAM else stream
-
-
-def launch_order(stream: int):
-    """Held while a call enqueues its launches on ``stream``: they use the stream's scratch,
-    and another thread's must not come in between."""
-    return _order[hash(_stream_key(stream)) % len(_order)]
-
-
-class LongFFT:
+class LongFFT(StreamScratch):
     """``count`` packed transforms of one length that split_length() cuts, in place in a
     complex64 buffer.  A batch of more than CHUNK_POINTS points runs in chunks of whole
     transforms, so that what lies between the launches stays in the cache."""
@@ -234,32 +217,7 @@ class LongFFT:
         self.tables = _twiddles(self.n, self.kernels[each][0].plan.radices[-1])
         # whole row tiles of the largest chunk (the tile of a smaller one may be narrower)
         self._points = max(c * scratch_points(self.n, k[1].plan.B) for c, k in self.kernels.items())
-        self._scratch: Dict[int, Buffer] = {}
-        self._captured: Dict[Tuple[int, int], Buffer] = {}
-        self._lock = threading.Lock()
-
-    def _scratch_for(self, stream: int) -> Buffer:
-        """The data between the launches of a call, one buffer per stream: calls on different
-        streams may overlap.  The plan keeps those of the last SCRATCH_STREAMS streams (a
-        further one frees the oldest, which waits for the GPU).  A call inside a capture of the
-        caller's takes a buffer that the plan keeps for this capture: its replays may run at
-        any time and on any stream."""
-        with self._lock:
-            if rt.is_capturing(stream):
-                return self._scratch_of_capture(stream)
-            key = _stream_key(stream)
-            s = self._scratch.pop(key, None) or self._new_scratch()
-            self._scratch[key] = s  # the newest comes last
-            while len(self._scratch) > SCRATCH_STREAMS:
-                del self._scratch[next(iter(self._scratch))]
-            return s
-
-    def _scratch_of_capture(self, stream: int) -> Buffer:
-        kept = self._captured = self._captured or {}
-        key = (rt.capture_id(stream), _stream_key(stream))  # the branches of one capture may overlap, too
-        if key not in kept:
-            kept[key] = self._new_scratch() if len(kept) < SCRATCH_CAPTURES else kept.pop(next(iter(kept)))
-        return kept[key]
+        self._init_scratch()
 
     def _new_scratch(self) -> Buffer:
         with rt.allocating_in_capture():  # launches may be recorded while a caller captures
