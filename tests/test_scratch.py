@@ -4,10 +4,12 @@ import threading
 
 import pytest
 
+from vkdispatch_amd import dtypes as dt
 from vkdispatch_amd import graph as G
 from vkdispatch_amd import runtime as rt
 from vkdispatch_amd.fft import functions as F
 from vkdispatch_amd.fft import long as LG
+from vkdispatch_amd.fft import scratch
 
 
 class _Kernel:
@@ -17,8 +19,14 @@ class _Kernel:
     def handle(self):
         return 1
 
+    def bind(self, values):
+        return [v.ptr for v in values], b""
+
+    def launch(self, values, stream):
+        self.launch_raw(*self.bind(values), stream)
+
     def launch_raw(self, ptrs, consts=b"", stream=None):
-        self.log.append((self.name, stream, tuple(ptrs)))
+        self.log.append((self.name, rt.current_stream() if stream is None else stream, tuple(ptrs)))
 
 
 class _Data:
@@ -43,6 +51,10 @@ def device(monkeypatch):
     monkeypatch.setattr(rt, "synchronize", lambda stream=None: None)
     monkeypatch.setattr(rt, "current_stream", lambda: dev.stream)
     monkeypatch.setattr(rt, "is_capturing", lambda s=None: (dev.stream if s is None else s) in dev.capturing)
+    monkeypatch.setattr(rt, "lib", lambda: dev)
+    dev.vkx_graph_begin = lambda s: dev.capturing.update({s: 1000 + s}) or 0
+    dev.vkx_graph_end = lambda s, h: dev.capturing.pop(s) and 0
+    dev.vkx_graph_launch = dev.vkx_graph_destroy = lambda *a: 0
     monkeypatch.setattr(rt, "capture_id", lambda s: dev.capturing.get(s, 0), raising=False)
     return dev
 
@@ -68,35 +80,59 @@ def _between(log):
     return out
 
 
-def _call(plan, monkeypatch, buf, graph=None):
+def _long(monkeypatch):
     """fft() of a long length as functions.py routes it."""
-    monkeypatch.setattr(F, "_uniform_plan", lambda *a: plan)
-    from vkdispatch_amd import dtypes as dt
-    assert F._large_or_prime_fallback((buf,), (3, 1 << 20), None, False, True, False, None, None, dt.complex64,
-                                      dt.complex64, None, graph)
-
-
-def test_recorded_long_transforms_share_nothing_with_calls(device, monkeypatch):
-    """Recorded on one stream and submitted on another beside calls on the first; two graphs
-    recorded on one stream and submitted on two; the launches of one graph share."""
     plan, log = _long_plan()
+    plan._init_scratch(64)
+    monkeypatch.setattr(F, "_uniform_plan", lambda *a: plan)
+
+    def call(buf, graph):
+        assert F._large_or_prime_fallback((buf,), (3, 1 << 20), None, False, True, False, None, None, dt.complex64,
+                                          dt.complex64, None, graph)
+    return plan, log, call, _between
+
+
+_Kinds = {"long": _long}
+
+
+@pytest.mark.parametrize("kind", ["long"])
+def test_recorded_launches_share_nothing_with_calls(device, monkeypatch, kind):
+    """Recorded on one stream and submitted on others beside calls on the first; two graphs
+    recorded on one stream and submitted on two: each stream its own, kept while a graph
+    may run with it."""
+    monkeypatch.setattr(scratch, "_streams", {})
+    monkeypatch.setattr(scratch, "_pinned", [])
+    plan, log, call, between = _Kinds[kind](monkeypatch)
     graphs = [G.CommandGraph(), G.CommandGraph()]
     for g in graphs:
-        for b in (100, 200):
-            _call(plan, monkeypatch, _Data(b), g)
+        for b in (1 << 25, 1 << 26):
+            call(_Data(b), g)
     assert not log
-    for g, s in zip(graphs, (2, 3)):
-        g._replay(s)
-    _call(plan, monkeypatch, _Data(300))
+    for g, s in zip(graphs, (5, 6)):
+        g.submit(stream=s)               # captured for s
+        assert g._exec_stream == s
+    call(_Data(1 << 27), None)
+    graphs[0].submit(stream=6, use_graph=False)
     used = {}
-    for s, y in _between(log):
+    for s, y in between(log):
         used.setdefault(s, set()).add(y)
-    assert sorted(used) == [1, 2, 3] and all(len(v) == 1 for v in used.values())
-    assert len(set.union(*used.values())) == 3
-    assert not device.freed
-    y2 = used[2]
-    graphs[0].reset()
-    assert set(device.freed) == y2
+    assert sorted(used) == [1, 5, 6] and all(len(v) == 1 for v in used.values())
+    outside = set.union(*used.values())
+    assert len(outside) == 3
+    del log[:]
+    device.capturing = {7: 9}            # into a capture of the caller's
+    for g in graphs:
+        g.submit(stream=7)
+    device.capturing = {}
+    inside = {y for _, y in between(log)}
+    assert len(inside) == 2 and not inside & outside
+    scratch._streams.clear()
+    assert set(device.freed) == used[1]  # the graphs hold theirs
+    for g in graphs:
+        g.reset()
+    assert set(device.freed) == outside  # and captured graphs what they were given
+    scratch.clear()
+    assert set(device.freed) == outside | inside
 
 
 def test_a_bound_long_transform_has_its_own_scratch(device):
@@ -170,12 +206,11 @@ def test_two_threads_on_one_stream_take_turns(device):
 
 def test_plans_on_one_stream_share_a_buffer(device, monkeypatch):
     """What calls keep grows with the largest plan and the streams, not with the plans."""
-    from vkdispatch_amd.fft import scratch
     monkeypatch.setattr(scratch, "_streams", {})
     plans = []
     for points in (64, 32, 128, 64):
         plan, log = _long_plan(points)
-        plan._init_scratch()
+        plan._init_scratch(points)
         plans.append((plan, log))
         plan(_Data(100))
     got = [_between(log)[0][1] for _, log in plans]

@@ -177,7 +177,10 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
     plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize))
     buf = buffers[0]
     if graph is not None and not graph.submit_on_record:
-        graph.record_callable(plan.bind(buf, graph=graph) if isinstance(plan, LongFFT) else plan.bind(buf))
+        if isinstance(plan, LongFFT):
+            plan.record(buf, graph)
+        else:
+            graph.record_callable(plan.bind(buf))
     else:
         plan(buf)
     return True

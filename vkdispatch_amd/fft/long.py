@@ -216,8 +216,7 @@ class LongFFT(StreamScratch):
             check_no_spill(k)
         self.tables = _twiddles(self.n, self.kernels[each][0].plan.radices[-1])
         # whole row tiles of the largest chunk (the tile of a smaller one may be narrower)
-        self._points = max(c * scratch_points(self.n, k[1].plan.B) for c, k in self.kernels.items())
-        self._init_scratch()
+        self._init_scratch(max(c * scratch_points(self.n, k[1].plan.B) for c, k in self.kernels.items()))
 
     def _new_scratch(self) -> Buffer:
         with rt.allocating_in_capture():  # launches may be recorded while a caller captures
@@ -235,13 +234,15 @@ class LongFFT(StreamScratch):
             calls += [(cols, [y.ptr, x, a.ptr, r.ptr]), (rows, [x, y.ptr])]
         return calls
 
-    def bind(self, buf, graph=None):
-        """``launch(stream)`` for this buffer; it allocates nothing (safe under graph capture)
-        and has scratch of its own, or that of the CommandGraph it is recorded into: it may
-        run on any stream, beside calls of this plan."""
+    def _load(self) -> None:
         for k in {k for pair in self.kernels.values() for k in pair}:
             k.handle()
-        y = self._new_scratch() if graph is None else graph.scratch(8 * self._points)
+
+    def bind(self, buf):
+        """``launch(stream)`` for this buffer; it allocates nothing (safe under graph capture)
+        and has scratch of its own: it may run on any stream, beside calls of this plan."""
+        self._load()
+        y = self._new_scratch()
         calls = self._launches(buf, y)
         keep = (buf, y, self)
 
@@ -251,9 +252,19 @@ class LongFFT(StreamScratch):
                 k.launch_raw(ptrs, b"", stream)
         return launch
 
+    def record(self, buf, graph) -> None:
+        """Into a CommandGraph that is submitted later."""
+        self._load()
+        self._launches(buf, buf)  # refused now, not when it is submitted
+
+        def launch(stream, y):
+            for k, ptrs in self._launches(buf, y):
+                k.launch_raw(ptrs, b"", stream)
+        graph.record_with_scratch(launch, self._points)
+
     def __call__(self, buf) -> None:
         stream = rt.current_stream()
-        with launch_order(stream):
+        with launch_order():
             y = self._scratch_for(stream)
             for k, ptrs in self._launches(buf, y):
                 k.launch_raw(ptrs, b"", stream)

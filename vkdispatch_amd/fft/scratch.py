@@ -5,10 +5,11 @@ It belongs to one sequence of launches at a time, so work that can overlap never
 * a call takes the buffer of its stream, which all plans share (work on a stream runs in
   order) and which grows to the largest of them; it holds ``launch_order`` while it
   enqueues, so that another thread's launches on that stream do not come in between;
-* launches that are kept and run later, on any stream, have a buffer of their own, or that of
-  the CommandGraph that they are recorded into (``CommandGraph.scratch``);
-* a call inside a capture of the caller's takes a buffer that its plan keeps for this
-  capture: the replays may run at any time and on any stream.
+* a CommandGraph takes that of the stream it is submitted on, when it is captured for it
+  (the graph then runs on this stream only);
+* inside a capture of the caller's, whose replays may run at any time and on any stream, a call
+  takes a buffer that its plan keeps for this capture, and a CommandGraph one that it keeps;
+* a launch that is bound to be run later, on any stream, has a buffer of its own.
 
 A buffer that is let go is freed by hipFree, which waits for the work in flight.
 """
@@ -18,6 +19,7 @@ import threading
 from typing import Dict, List, Tuple
 
 from .. import runtime as rt
+from ..buffer import Buffer
 from .shader_factories import register_plan_cache
 
 SCRATCH_STREAMS = 6    # streams whose buffers are kept; while calls alternate between more, each frees the
@@ -28,34 +30,33 @@ SCRATCH_CAPTURES = 16  # captures of a plan with a buffer of their own; the next
 _streams: Dict[object, Tuple[int, object]] = {}
 _streams_lock = threading.Lock()
 _pinned: List[object] = []
-_order = [threading.RLock() for _ in range(16)]
-_PER_THREAD_STREAM = 2  # hipStreamPerThread: one handle for a stream of each thread
+_order = threading.RLock()
 
 
-def _stream_key(stream: int):
-    return (stream, threading.get_ident()) if stream == _PER_THREAD_STREAM else stream
-
-
-def launch_order(stream: int):
-    """Held while a call enqueues its launches on ``stream``: they use the stream's scratch,
-    and another thread's must not come in between."""
-    return _order[hash(_stream_key(stream)) % len(_order)]
+def launch_order():
+    """Held while a call enqueues launches that use its stream's scratch: another thread's on
+    this stream must not come in between."""
+    return _order
 
 
 class StreamScratch:
-    """A plan with ``_points`` complex64 values between its launches; ``_new_scratch()`` allocates
-    them."""
+    """Owner of launches with ``_points`` complex64 values between them."""
 
-    def _init_scratch(self) -> None:
+    def _init_scratch(self, points: int) -> None:
+        self._points = int(points)
         self._scratch, self._lock = _streams, _streams_lock
         self._captured: Dict[tuple, object] = {}
 
+    def _new_scratch(self) -> Buffer:
+        with rt.allocating_in_capture():
+            return Buffer((self._points,))
+
     def _scratch_for(self, stream: int):
-        """The buffer of a call on ``stream``, to be used under ``launch_order(stream)``."""
+        """The buffer of a call on ``stream``, to be used under ``launch_order()``."""
         with self._lock:
             if rt.is_capturing(stream):
                 return self._scratch_of_capture(stream)
-            key = _stream_key(stream)
+            key = rt.stream_key(stream)
             have = self._scratch.pop(key, None)
             if have is None or have[0] < self._points:
                 have = (self._points, self._new_scratch())
@@ -66,16 +67,19 @@ class StreamScratch:
 
     def _scratch_of_capture(self, stream: int):
         kept = self._captured = self._captured or {}
-        key = (rt.capture_id(stream), _stream_key(stream))  # the branches of one capture may overlap, too
+        # the branches of one capture may overlap, too
+        key = (rt.capture_id(stream), rt.stream_key(stream), self._points)
         if key not in kept:
-            kept[key] = self._new_scratch() if len(kept) < SCRATCH_CAPTURES else kept.pop(next(iter(kept)))
+            full = len(kept) >= SCRATCH_CAPTURES
+            oldest = next((k for k in kept if k[2] >= self._points), None) if full else None
+            kept[key] = self._new_scratch() if oldest is None else kept.pop(oldest)
             if self not in _pinned:
                 _pinned.append(self)  # a plan cache may drop the plan; the captured graph needs its memory
         return kept[key]
 
 
 def clear() -> None:
-    """Let go of the buffers of calls and captures (graphs and bound launches keep theirs)."""
+    """Let go of the buffers of calls and captures (graphs and bound launches hold theirs)."""
     with _streams_lock:
         _streams.clear()
         _pinned.clear()

@@ -24,9 +24,10 @@ class CommandGraph:
         self.submit_on_record = submit_on_record
         # (kernel or launcher, device pointers, packed constants, objects kept alive)
         self._records: List[Tuple[object, Optional[List[int]], Optional[bytes], tuple]] = []
-        self._scratch: List[object] = []
+        self._scratch = None  # StreamScratch of the records that need one
         self._exec: Optional[int] = None
-        self._exec_stream: Optional[int] = None
+        self._exec_stream = None
+        self._exec_scratch = None
 
     def record_kernel(self, kernel, values) -> None:
         ptrs, consts = kernel.bind(values)
@@ -49,16 +50,17 @@ class CommandGraph:
         self._records.append((fn, None, None, ()))
         self._drop_exec()
 
-    def scratch(self, nbytes: int):
-        """A buffer of at least ``nbytes`` for what recorded launches hand to each other.  The
-        launches of a graph run one after another, so they share it; nothing else uses it."""
-        for b in self._scratch:
-            if b.mem_size >= nbytes:
-                return b
-        from .buffer import Buffer
-        with rt.allocating_in_capture():  # launches may be recorded while a caller captures
-            self._scratch.append(Buffer((-(-int(nbytes) // 8),)))
-        return self._scratch[-1]
+    def record_with_scratch(self, fn, points: int) -> None:
+        """Record a launcher ``fn(stream, scratch)`` whose launches hand ``points`` complex64
+        values to each other.  All of a graph's share one buffer (they run one after
+        another), that of the stream the graph runs on (fft/scratch.py)."""
+        if self._scratch is None:
+            from .fft.scratch import StreamScratch
+            self._scratch = StreamScratch()
+            self._scratch._init_scratch(points)
+        self._scratch._points = max(self._scratch._points, int(points))
+        self._records.append((fn, (), None, ()))
+        self._drop_exec()
 
     def __len__(self):
         return len(self._records)
@@ -66,26 +68,40 @@ class CommandGraph:
     def _drop_exec(self):
         if self._exec is not None:
             rt.lib().vkx_graph_destroy(self._exec)
-            self._exec = None
+            self._exec = self._exec_scratch = None
 
-    def _replay(self, stream: int) -> None:
+    def _scratch_on(self, stream: int):
+        return None if self._scratch is None else self._scratch._scratch_for(stream)
+
+    def _replay(self, stream: int, scratch=None) -> None:
         for k, ptrs, consts, _keep in self._records:
             if ptrs is None:
                 k(stream)
+            elif consts is None:
+                k(stream, scratch)
             else:
                 k.launch_raw(ptrs, consts, stream)
 
+    def _replay_now(self, stream: int) -> None:
+        if self._scratch is None:
+            self._replay(stream)
+            return
+        from .fft.scratch import launch_order
+        with launch_order():
+            self._replay(stream, self._scratch_on(stream))
+
     def capture(self, stream: Optional[int] = None) -> int:
         s = rt.current_stream() if stream is None else int(stream)
-        if self._exec is None or self._exec_stream != s:
+        if self._exec is None or self._exec_stream != rt.stream_key(s):
             self._drop_exec()
+            scratch = self._scratch_on(s)  # before the capture: the stream's own
             rt.check(rt.lib().vkx_graph_begin(s), "vkx_graph_begin")
             try:
-                self._replay(s)
+                self._replay(s, scratch)
             finally:
                 h = ctypes.c_uint64(0)
                 rt.check(rt.lib().vkx_graph_end(s, ctypes.byref(h)), "vkx_graph_end")
-            self._exec, self._exec_stream = h.value, s
+            self._exec, self._exec_stream, self._exec_scratch = h.value, rt.stream_key(s), scratch
         return self._exec
 
     def submit(self, instance_count: Optional[int] = None, queue_index: int = -2, stream=None,
@@ -101,21 +117,21 @@ class CommandGraph:
             # the caller is capturing this stream (torch.cuda.graph): launch the records
             # directly so that they become nodes of the caller's graph
             for _ in range(reps):
-                self._replay(s)
+                self._replay_now(s)
         elif use_graph:
             ex = self.capture(s)
             for _ in range(reps):
                 rt.check(rt.lib().vkx_graph_launch(ex, s), "vkx_graph_launch")
         else:
             for _ in range(reps):
-                self._replay(s)
+                self._replay_now(s)
         if self.reset_on_submit:
             self.reset()
 
     def reset(self) -> None:
         self._drop_exec()
         self._records = []
-        self._scratch = []
+        self._scratch = None
 
     def destroy(self) -> None:
         self.reset()

@@ -320,6 +320,12 @@ def is_capturing(stream=None) -> bool:
     return c.value != 0
 
 
+def stream_key(stream: int):
+    """What tells streams apart: the handle, but hipStreamPerThread (2) is a stream of each
+    thread's under one handle."""
+    return (stream, threading.get_ident()) if stream == 2 else stream
+
+
 def capture_id(stream: int) -> int:
     """A number that tells the captures under way on ``stream`` apart (0: none)."""
     if not device_initialised():
