@@ -8,6 +8,7 @@ from vkdispatch_amd import dtypes as dt
 from vkdispatch_amd import graph as G
 from vkdispatch_amd import runtime as rt
 from vkdispatch_amd.fft import functions as F
+from vkdispatch_amd.fft import fused as FU
 from vkdispatch_amd.fft import long as LG
 from vkdispatch_amd.fft import scratch
 
@@ -92,10 +93,32 @@ def _long(monkeypatch):
     return plan, log, call, _between
 
 
-_Kinds = {"long": _long}
+def _conv(monkeypatch):
+    """convolve2DR of square images."""
+    log = []
+    plan = FU.Conv2DPhases(3, 256, 256)
+    plan.kernels_ = [_Kernel(log, n) for n in ("rows", "cols", "irows")]
+    plan._checked = True
+    monkeypatch.setattr(FU, "fused_eligible", lambda *a, **kw: plan)
+
+    def call(buf, graph):
+        assert FU.try_convolve2DR(buf, _Data(77), graph)
+
+    def between(log):
+        out = []
+        for three in zip(log[::3], log[1::3], log[2::3]):
+            assert [n for n, _, _ in three] == ["rows", "cols", "irows"]
+            (key,) = {(s, p[2]) for _, s, p in three}
+            assert all(p[1] == 77 and p[5] == p[2] + 8 * 2 * 256 * 256 for _, _, p in three)  # two pairs, then Kt
+            out.append(key)
+        return out
+    return plan, log, call, between
 
 
-@pytest.mark.parametrize("kind", ["long"])
+_Kinds = {"long": _long, "conv": _conv}
+
+
+@pytest.mark.parametrize("kind", ["long", "conv"])
 def test_recorded_launches_share_nothing_with_calls(device, monkeypatch, kind):
     """Recorded on one stream and submitted on others beside calls on the first; two graphs
     recorded on one stream and submitted on two: each stream its own, kept while a graph
@@ -168,6 +191,26 @@ def test_captures_share_nothing(device):
         device.stream = 1
         used(plan, _Data(300))
     assert len(plan._captured) == LG.SCRATCH_CAPTURES and not set(device.freed) & set(first)
+
+
+def test_two_threads_convolve_in_turn(device, monkeypatch):
+    monkeypatch.setattr(scratch, "_streams", {})
+    plan, log, call, between = _conv(monkeypatch)
+    inside, other = threading.Event(), threading.Event()
+
+    class Slow(_Kernel):
+        def launch_raw(self, ptrs, consts=b"", stream=None):
+            super().launch_raw(ptrs, consts, stream)
+            if not inside.is_set():
+                inside.set()
+                other.wait(0.3)
+    plan.kernels_[0] = Slow(log, "rows")
+    t = threading.Thread(target=lambda: (inside.wait(), call(_Data(1 << 26), None), other.set()))
+    t.start()
+    call(_Data(1 << 25), None)
+    t.join()
+    between(log)
+    assert [p[0] for _, _, p in log] == [1 << 25] * 3 + [1 << 26] * 3
 
 
 def test_two_threads_on_one_stream_take_turns(device):

@@ -14,18 +14,18 @@ VKX_FUSED_CONV=0 forces the three-dispatch composition.
 from __future__ import annotations
 
 import os
-import threading
 from functools import lru_cache
 from typing import Dict, List, Optional, Sequence, Tuple
 
 from .. import dtypes as dt
 from .. import runtime as rt
 from ..buffer import Buffer
-from ..graph import dispatch
+from ..graph import CommandGraph, dispatch
 from . import half2d
 from .hooks import Arg
 from .kernels import CompiledKernel, SpillError, check_no_spill, kernel_symbol, source_symbol
 from .planner import KernelPlan
+from .scratch import StreamScratch, launch_order
 from .shader_factories import make_convolution_shader, make_fft_shader, register_plan_cache
 
 _FUSED_RADICES = {256: (4, 4, 4, 4), 512: (8, 8, 8), 1024: (16, 16, 4)}
@@ -93,11 +93,11 @@ def _conv_tu(cfg: str, symbol: str, block: int, waves_per_simd: Optional[int], b
                       f"  {body}", "}", ""])
 
 
-class Conv2DPhases:
+class Conv2DPhases(StreamScratch):
     """The same computation as three ordinary kernels in stream order: row FFTs of the
     image pairs (plus the kernel prep), column FFT * Kt * IFFT, row IFFTs; each pair's
     spectrum goes through a column-major scratch image (64 MiB for 64 images of
-    512 x 512) and Kt is one 512 x 512 complex image."""
+    512 x 512) and Kt is one 512 x 512 complex image (who shares them: fft/scratch.py)."""
 
     def __init__(self, batch: int, H: int, W: int, normalize: bool = True, waves: int = 8, rows: int = 16,
                  col_waves: int = 8, layout: str = "column", cols_per_wave: int = 1, pairs_per_task: int = 4,
@@ -134,36 +134,38 @@ class Conv2DPhases:
             radices = list(plan.radices)
             self.kernels_.append(CompiledKernel(src, plan, args, radices, radices[::-1],
                                                 name=f"conv2d_{tag}_{batch}x{H}x{W}"))
-        self._dev: Optional[Tuple[Buffer, Buffer]] = None
+        # one pair image per two images, and behind them Kt
+        self._init_scratch((self.npairs + 1) * self.H * self.W)
         self._checked = False
-        self._lock = threading.Lock()
 
     def kernels(self) -> List[CompiledKernel]:
         return list(self.kernels_)
 
-    def resources(self) -> Tuple[Buffer, Buffer]:
-        if self._dev is None:
-            with self._lock:
-                if self._dev is None:
-                    rt.require_not_capturing("the first call of a 2-D convolution plan")
-                    self._dev = (Buffer((self.npairs * self.H, self.W), dt.complex64),
-                                 Buffer((self.H, self.W), dt.complex64))
-        return self._dev
-
-    def scratch(self) -> Buffer:
-        return self.resources()[0]
-
-    def values(self, buffer, kernel) -> list:
+    def values(self, buffer, kernel, scratch=None) -> list:
+        """The kernels' arguments, through ``scratch`` (default: that of the current stream's
+        calls)."""
         if not self._checked:
             _check_no_spill(self.kernels())
             self._checked = True
-        scr, kt = self.resources()
+        scr = self._scratch_for(rt.current_stream()) if scratch is None else scratch
+        kt = Buffer((self.H, self.W), dt.complex64, external=(scr.ptr + 8 * self.npairs * self.H * self.W, scr, True))
         return [buffer, kernel, scr, scr, scr, kt]
 
     def __call__(self, buffer, kernel, graph=None) -> None:
-        vals = self.values(buffer, kernel)
-        for k in self.kernels_:
-            dispatch(k, vals, graph)
+        if isinstance(graph, CommandGraph) and not graph.submit_on_record:
+            for k in self.kernels_:
+                k.handle()
+
+            def launch(stream, scratch):
+                vals = self.values(buffer, kernel, scratch)
+                for k in self.kernels_:
+                    k.launch(vals, stream)
+            graph.record_with_scratch(launch, self._points)
+            return
+        with launch_order():
+            vals = self.values(buffer, kernel)
+            for k in self.kernels_:
+                dispatch(k, vals, graph)
 
 
 # phase-kernel tilings: for 512 the row kernels run one row per wave (16 waves, 64 VGPRs,
@@ -247,9 +249,10 @@ def try_convolve2DR(buffer, kernel, graph=None, print_shader=False, **kw) -> boo
     if print_shader:
         for k in plan.kernels():
             print(k.source)
-    vals = plan.values(buffer, kernel)
-    for k in plan.kernels():
-        dispatch(k, vals, graph)
+    if isinstance(plan, Conv2DPhases):
+        plan(buffer, kernel, graph)
+    else:
+        dispatch(plan.kernel, plan.values(buffer, kernel), graph)
     return True
 
 
