@@ -10,6 +10,7 @@ from vkdispatch_amd import runtime as rt
 from vkdispatch_amd.fft import functions as F
 from vkdispatch_amd.fft import fused as FU
 from vkdispatch_amd.fft import long as LG
+from vkdispatch_amd.fft import mixed as MX
 from vkdispatch_amd.fft import scratch
 
 
@@ -115,10 +116,36 @@ def _conv(monkeypatch):
     return plan, log, call, between
 
 
-_Kinds = {"long": _long, "conv": _conv}
+def _mixed(monkeypatch, passes=2):
+    """fft3_mixed, two passes with one volume between them or three with two."""
+    log = []
+    plan = MX.Mixed3D((256, 256, 256), dt.complex_bf16, passes=passes)
+    plan.passes = [_Kernel(log, str(n)) for n in range(passes)]
+    monkeypatch.setattr(MX, "_plan", lambda *a: plan)
+
+    def call(buf, graph):
+        out = _Data(buf.ptr + 8)
+        buf.shape = out.shape = (256, 256, 256)
+        buf.var_type, out.var_type = dt.complex_bf16, dt.complex64
+        MX.fft3_mixed(out, buf, graph=graph)
+
+    def between(log):
+        got = []
+        for group in zip(*[log[i::passes] for i in range(passes)]):
+            assert [n for n, _, _ in group] == [str(n) for n in range(passes)]
+            assert all(a[2][0] == b[2][1] for a, b in zip(group, group[1:]))  # each reads what the last wrote
+            assert group[-1][2][0] == group[0][2][1] + 8
+            ((s, y),) = {(s, group[0][2][0]) for _, s, _ in group}
+            assert passes == 2 or group[1][2][0] == y + 4 * 256 ** 3 < y + 8 * plan._points
+            got.append((s, y))
+        return got
+    return plan, log, call, between
 
 
-@pytest.mark.parametrize("kind", ["long", "conv"])
+_Kinds = {"long": _long, "conv": _conv, "mixed": _mixed, "mixed3": lambda m: _mixed(m, 3)}
+
+
+@pytest.mark.parametrize("kind", ["long", "conv", "mixed", "mixed3"])
 def test_recorded_launches_share_nothing_with_calls(device, monkeypatch, kind):
     """Recorded on one stream and submitted on others beside calls on the first; two graphs
     recorded on one stream and submitted on two: each stream its own, kept while a graph

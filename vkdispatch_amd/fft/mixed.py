@@ -21,7 +21,7 @@ from __future__ import annotations
 
 import os
 from functools import lru_cache
-from typing import Optional, Tuple
+from typing import Optional
 
 from .. import dtypes as dt
 from .. import runtime as rt
@@ -30,6 +30,7 @@ from ..graph import CommandGraph, dispatch
 from .hooks import Arg
 from .kernels import CompiledKernel, kernel_symbol, translation_unit
 from .planner import KernelPlan
+from .scratch import StreamScratch, launch_order
 from .shader_factories import register_plan_cache
 
 _SCALAR_CPP = {dt.complex_bf16: "vkx::bf16", dt.complex32: "_Float16", dt.complex64: "float"}
@@ -109,7 +110,7 @@ def make_cube_pass(which: int, in_type, inverse: bool = False, out_scale: float 
     return CompiledKernel(src, plan, args, None, None, name=f"mfma3d_p{which}", roots_n=256)
 
 
-class Mixed3D:
+class Mixed3D(StreamScratch):
     """Plan for the 3-D mixed-precision transform of one 256 x 256 x 256 volume, complex64
     result in natural order.  ``passes=2`` (default): the two-pass form, 16-bit input ->
     fp16 intermediate -> complex64 (three radix-16 MFMA stages per pass); ``run`` = 4 or 8
@@ -153,7 +154,8 @@ class Mixed3D:
                 make_tw_pass(nb, mid, mid, inverse, s_mid, T16, block),
                 make_tw_pass(nb, mid, dt.complex64, inverse, 256.0 * norm, None, block),
             ]
-        self._scratch: Optional[Tuple[Buffer, Buffer]] = None
+        # 16-bit volumes between the passes: one, or two in turn
+        self._init_scratch((1 if passes == 2 else 2) * 256 ** 3 // 2)
 
     def kernels(self):
         return list(self.passes)
@@ -169,26 +171,33 @@ class Mixed3D:
         cubes = 4096  # 16 x 16 x 16 blocks per pass, 16 tiles + 16 cross tiles each
         return cubes * (16 * tile + 16 * 4) + cubes * (16 * tile + 16 * (4 if self.half_tiles_p2 else 6))
 
-    def scratch(self) -> Tuple[Buffer, ...]:
-        if self._scratch is None:
-            n = 1 if self.npasses == 2 else 2
-            self._scratch = tuple(Buffer(self.shape, dt.complex32) for _ in range(n))
-        return self._scratch
+    def _steps(self, out: Buffer, inp: Buffer, scratch: Buffer) -> list:
+        """(kernel, arguments) of every pass through ``scratch``."""
+        if self.npasses == 2:
+            return [(self.passes[0], [scratch, inp]),     # -> M[c1][k2/4][i0][a1][k2%4]
+                    (self.passes[1], [out, scratch])]     # -> [k0][k1][k2]
+        second = Buffer(self.shape, dt.complex32, external=(scratch.ptr + 4 * 256 ** 3, scratch, True))
+        return [(self.passes[0], [scratch, inp]),         # [i0][i1][i2] -> [k2][i0][i1]
+                (self.passes[1], [second, scratch]),      # -> [k1][k2][i0]
+                (self.passes[2], [out, second])]          # -> [k0][k1][k2]
 
     def __call__(self, out: Buffer, inp: Buffer, graph: Optional[CommandGraph] = None) -> None:
         if out.var_type is not dt.complex64 or tuple(out.shape) != self.shape:
             raise ValueError("output must be a complex64 buffer of the volume's shape")
         if inp.var_type is not self.in_type or tuple(inp.shape) != self.shape:
             raise ValueError(f"input must be a {self.in_type.name} buffer of the volume's shape")
-        if self.npasses == 2:
-            (m,) = self.scratch()
-            dispatch(self.passes[0], [m, inp], graph)    # -> M[c1][k2/4][i0][a1][k2%4]
-            dispatch(self.passes[1], [out, m], graph)    # -> [k0][k1][k2]
+        if isinstance(graph, CommandGraph) and not graph.submit_on_record:
+            for k in self.passes:
+                k.handle()
+
+            def launch(stream, scratch):
+                for k, vals in self._steps(out, inp, scratch):
+                    k.launch(vals, stream)
+            graph.record_with_scratch(launch, self._points)
             return
-        s1, s2 = self.scratch()
-        dispatch(self.passes[0], [s1, inp], graph)   # [i0][i1][i2] -> [k2][i0][i1]
-        dispatch(self.passes[1], [s2, s1], graph)    # -> [k1][k2][i0]
-        dispatch(self.passes[2], [out, s2], graph)   # -> [k0][k1][k2]
+        with launch_order():
+            for k, vals in self._steps(out, inp, self._scratch_for(rt.current_stream())):
+                dispatch(k, vals, graph)
 
 
 @lru_cache(maxsize=8)
