@@ -253,7 +253,7 @@ def _autograd_function():
 
     class FFTConvolve2DFunction(torch.autograd.Function):
         @staticmethod
-        def forward(ctx, x, k):
+        def forward(ctx, x, k, recorded):
             shape = x.shape
             H, W = shape[-2], shape[-1]
             if tuple(k.shape) != (H, W):
@@ -264,7 +264,8 @@ def _autograd_function():
             x3 = x.contiguous().reshape(-1, H, W)
             kc = k.contiguous()
             plans = plans_for(x3.shape[0], H, W, ctype)
-            y, K, kept = _run(_forward, x3, kc, plans, ctx.needs_input_grad[1])
+            y, K, kept = _run(_forward, x3, kc, plans,
+                              recorded and ctx.needs_input_grad[1])
             ctx.save_for_backward(kept, K)
             ctx.plans = plans
             ctx.in_shape = shape
@@ -278,7 +279,7 @@ def _autograd_function():
             dx, dk = _run(_backward, kept, K, g3, plans, ctx.needs_input_grad[0], ctx.needs_input_grad[1])
             if dx is not None:
                 dx = dx.reshape(ctx.in_shape)
-            return dx, dk
+            return dx, dk, None
 
     return FFTConvolve2DFunction
 
@@ -292,10 +293,8 @@ def fft_convolve2d(x, k):
     global _FN
     if _FN is None:
         _FN = _autograd_function()
-    torch = _torch()
-    if not torch.is_grad_enabled() and isinstance(k, torch.Tensor):
-        k = k.detach()  # no backward pass: nothing is kept for the gradient of k
-    return _FN.apply(x, k)
+    # where no backward pass is recorded nothing is kept for the gradient of k
+    return _FN.apply(x, k, _torch().is_grad_enabled())
 
 
 def FFTConvolve2D(H: int, W: int, dtype=None, init_std: float = 0.01):
