@@ -38,3 +38,31 @@ def test_forward_mode_is_refused(kept, which, recorded):
         args[which] = fwd_ad.make_dual(args[which], torch.ones_like(args[which]))
         with pytest.raises(NotImplementedError):
             autograd.fft_convolve2d(*args)
+
+
+def test_launches_that_spill_have_one_that_does_not(monkeypatch):
+    """plans_for compiles the launches that do all of the work; where one that does a part of it
+    would spill, theirs take its place."""
+    from vkdispatch_amd import dtypes as dt
+    from vkdispatch_amd.fft.kernels import SpillError
+    plan = autograd._HalfPlans(2, 64, 48, dt.complex64)
+    ran, spilling = [], set()
+
+    def check(kernel):
+        if kernel in spilling:
+            raise SpillError(kernel.name)
+    monkeypatch.setattr(autograd, "check_no_spill", check)
+    for name in ("conv", "conv_keep", "conv_dx", "grad", "rows_inv"):
+        monkeypatch.setattr(getattr(plan, name), "launch", lambda v, name=name: ran.append((name, v)))
+    x = torch.zeros(2, 64, 48)
+    ws = autograd._wrap(autograd._spectra(plan, 2, "cpu"), plan.ctype)
+    plan.forward(x, ws, ws, False)
+    plan.backward(None, ws, x, ws, True, False)
+    assert [n for n, _ in ran] == ["conv", "conv_dx", "rows_inv"]
+    plan._fits.clear()
+    ran.clear()
+    spilling |= {plan.conv, plan.conv_dx}
+    assert plan.forward(x, ws, ws, False) is None
+    dx, dk = plan.backward(None, ws, x, ws, True, False)
+    assert [n for n, _ in ran] == ["conv_keep", "grad", "rows_inv"] and dk is None and dx.shape == x.shape
+    assert len(ran[0][1]) == 3 and ran[1][1][1] is ws and ran[1][1][3].size == plan.grad.groups * 64 * 24

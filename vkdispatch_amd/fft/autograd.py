@@ -142,6 +142,18 @@ class _HalfPlans:
         self.conv_dx = half2d.make_half_conv(B, H, M, c, conj=False)
         self.grad = half2d.make_half_grad(B, H, M, c)
         self.rows_inv1 = make_real_rows_shader((1, H, W), True, True, c, c, True, W, M, True)
+        self._fits = {}
+
+    def fits(self, kernel) -> bool:
+        """Whether a launch that does part of another's work compiles without spills, found out
+        when it is first wanted (plans_for has compiled the others)."""
+        if kernel not in self._fits:
+            try:
+                check_no_spill(kernel)
+                self._fits[kernel] = True
+            except SpillError:
+                self._fits[kernel] = False
+        return self._fits[kernel]
 
     def kernels(self):
         return [self.rows_fwd, self.rows_inv, self.rows_fwd1, self.col_fft1, self.conv, self.conv_keep,
@@ -150,20 +162,21 @@ class _HalfPlans:
     def forward(self, x, ws, K, keep):
         """Columns of ws; returns what the gradient of k needs of x: its transform, which the
         column kernel has at hand.  It takes the place of x between the passes."""
-        if not keep:
+        if not keep and self.fits(self.conv):
             self.conv.launch([ws, K])
             return None
         X = _spectra(self, self.B, x.device)
         self.conv_keep.launch([ws, K, _wrap(X, self.ctype)])
-        return X
+        return X if keep else None
 
     def backward(self, X, K, g, Gb, need_dx, need_dk):
         torch = _torch()
         dx = dk = None
-        if need_dk:
+        if need_dk or not self.fits(self.conv_dx):
             partial = _wrap(_spectra(self, self.grad.groups, g.device), self.ctype)
-            self.grad.launch([Gb, _wrap(X, self.ctype), K, partial])
-        elif need_dx:
+            # where dk is not wanted its sum is of anything: of G
+            self.grad.launch([Gb, _wrap(X, self.ctype) if need_dk else Gb, K, partial])
+        else:
             self.conv_dx.launch([Gb, K])
         if need_dx:
             dx = torch.empty_like(g)
