@@ -20,6 +20,7 @@ from . import hooks
 from .kernels import CompiledKernel, cfg_struct, translation_unit
 from .planner import AxisGeometry, make_plan
 from .precision import kernel_real_type
+from .shader_factories import with_roomier
 
 
 class _Registers:
@@ -74,17 +75,20 @@ class FFTContext:
             raise ValueError("fft_context needs a read phase, execute() and a write phase")
         N = self.geom.N
         inv = self._inverse
-        cfg = cfg_struct(self.plan, in_os=N * self.geom.S, out_os=N * self.geom.S, k_os=N * self.geom.S,
-                         sig=(0, N), r2c=False, inverse=inv, normalize=inv and self._normalize, scale=1.0 / N)
         fin = ["struct HookIn {", "  template <class Op>",
                "  __device__ __forceinline__ static void apply(Op& op, const vkx::KParams& prm) {",
                *self._in_lines, "  }", "};"]
         fout = ["struct HookOut {", "  template <int K, class Op>",
                 "  __device__ __forceinline__ static void apply(Op& op, const vkx::KParams& prm) {",
                 *self._out_lines, "  }", "};"]
-        src = translation_unit(cfg, ["\n".join(fin), "\n".join(fout)], "vkx::fft_body<Cfg, HookIn, HookOut>(prm);",
-                               self.plan.BLOCK, "vkx_fft_context")
-        self._kernel = _ContextKernel(src, self.plan, self.args, list(self.plan.radices), None, name=self.name)
+
+        def build(plan):
+            cfg = cfg_struct(plan, in_os=N * self.geom.S, out_os=N * self.geom.S, k_os=N * self.geom.S, sig=(0, N),
+                             r2c=False, inverse=inv, normalize=inv and self._normalize, scale=1.0 / N)
+            src = translation_unit(cfg, ["\n".join(fin), "\n".join(fout)],
+                                   "vkx::fft_body<Cfg, HookIn, HookOut>(prm);", plan.BLOCK, "vkx_fft_context")
+            return _ContextKernel(src, plan, self.args, list(plan.radices), None, name=self.name)
+        self._kernel = with_roomier(build, self.plan, self.geom, "fft")
         return self._kernel
 
 

@@ -15,7 +15,7 @@ import hashlib
 import os
 import re
 import threading
-from typing import Dict, List, Optional, Sequence, Tuple
+from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
 
 import numpy as np
 
@@ -229,7 +229,7 @@ class CompiledKernel:
 
     def __init__(self, source: str, plan: KernelPlan, args, twiddle_fwd: Optional[List[int]],
                  twiddle_inv: Optional[List[int]], name: str = "vkx_fft", roots_n: int = 0):
-        self.plan = plan
+        self._plan = plan
         self.args = list(args)
         self.name = name
         self.tw_fwd = twiddle_fwd
@@ -238,15 +238,49 @@ class CompiledKernel:
         # The translation unit describes its own launch in its first line, so a backend
         # that receives only the source (the reference's stage_compute_plan_create)
         # can bind the same geometry and twiddle tables (launch_metadata()).
-        self.source = launch_comment(self.launch_metadata(source)) + source
+        self._source = launch_comment(self.launch_metadata(source)) + source
+        # () -> kernels of plans with fewer values a thread, the fastest first, should this
+        # one need private memory (settle)
+        self.roomier: Optional[Callable[[], Iterable["CompiledKernel"]]] = None
+        self._settling = threading.RLock()
         self._plan_handle = None
         self._lock = threading.Lock()
         self._buffers_only = all(a.kind == "buffer" for a in self.args)
 
+    def settle(self) -> None:
+        """Compile, and take the first roomier plan that needs no private memory if this one
+        does (how many registers a kernel needs, and whether its arrays stay in them, only the
+        compiler knows).  If all do it stays as it is, to be refused at its launch."""
+        if self.roomier is None:
+            return
+        with self._settling:
+            if self.roomier is None:
+                return
+            try:
+                if code_object_info(compile_source(self._source))["private_bytes"]:
+                    for k in self.roomier():
+                        if not code_object_info(compile_source(k._source))["private_bytes"]:
+                            self._plan, self._source, self.tw_fwd, self.tw_inv = k._plan, k._source, k.tw_fwd, k.tw_inv
+                            break
+            except RuntimeError:  # does not compile: its launch says so
+                pass
+            self.roomier = None
+
+    @property
+    def plan(self) -> KernelPlan:
+        self.settle()
+        return self._plan
+
+    @property
+    def source(self) -> str:
+        self.settle()
+        return self._source
+
     def launch_metadata(self, source: Optional[str] = None) -> Dict:
+        plan = self._plan if source is not None else self.plan
         return {"symbol": source_symbol(source if source is not None else self.source),
-                "grid": [int(v) for v in self.plan.grid], "block": [int(self.plan.BLOCK), 1, 1],
-                "n": int(self.plan.N), "double": 1 if self.plan.real == "double" else 0,
+                "grid": [int(v) for v in plan.grid], "block": [int(plan.BLOCK), 1, 1],
+                "n": int(plan.N), "double": 1 if plan.real == "double" else 0,
                 "radices_fwd": [int(r) for r in (self.tw_fwd or [])],
                 "radices_inv": [int(r) for r in (self.tw_inv or [])],
                 "roots_n": self.roots_n,
@@ -407,7 +441,7 @@ def precompile(kernels, workers: int = 0) -> int:
     from concurrent.futures import ThreadPoolExecutor
     srcs = []
     for k in kernels:
-        s = k if isinstance(k, str) else k.source
+        s = k if isinstance(k, str) else k._source  # in parallel, before settle() looks at it
         if not os.path.exists(os.path.join(cache_dir(), source_key(s) + ".hsaco")):
             srcs.append(s)
     srcs = list(dict.fromkeys(srcs))

@@ -91,12 +91,16 @@ def balanced_plan(N: int, elem: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     return None if best is None else best[1:]
 
 
+# values a thread may hold two sets of without spills, in workgroups of 513 to 1024, 257 to
+# 512 and up to 256 threads (128, 256 and 512 registers; 2556 kernels of 142 lengths compiled)
+_MOST_OF_TWO = ((13, 23, 32), (7, 14, 28))
 UNEVEN_LDS = 44 * 1024  # up to here enough workgroups share a CU to even its four SIMDs out
 
 
 @lru_cache(maxsize=None)
-def column_radices(N: int, elem: int, B: int) -> Optional[Tuple[Tuple[int, ...], int]]:
-    """(radices, threads per transform) of strided transforms, B of them in a workgroup: the
+def column_radices(N: int, elem: int, B: int, live: int = 1) -> Optional[Tuple[Tuple[int, ...], int]]:
+    """(radices, threads per transform) of strided transforms, B of them in a workgroup, that
+    hold ``live`` sets of values at once: the
     cost of balanced_plan without what only concerns contiguous rows, the smaller radices
     first (512 = 16 32 points 8.9 us, 32 16 9.9; 320 columns, 50 MB in and out).  The idle
     lanes are those of the workgroup's last wave: 96 points 6 16 8.7 us, 8 12 7.5.  Two or
@@ -117,6 +121,8 @@ def column_radices(N: int, elem: int, B: int) -> Optional[Tuple[Tuple[int, ...],
                 if tt * B > MAX_THREADS or values > max(most, max(rads)) or values < 4:
                     continue
                 if tt * B > 512 and values > (12 if dbl else 20):  # at most 128 registers
+                    continue
+                if live > 1 and values > _MOST_OF_TWO[dbl][0 if tt * B > 512 else 1 if tt * B > 256 else 2]:
                     continue
                 lanes = -(-tt * B // WAVE) * WAVE / (tt * B)
                 work = sum(slots(N, r, tt) * tt for r in rads) / N * lanes
@@ -291,12 +297,13 @@ def lookup(geom: AxisGeometry, real: str, kind: str) -> Optional[dict]:
 def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int] = None,
               radices: Optional[List[int]] = None, tt: Optional[int] = None,
               need_lds: bool = False, kind: str = "fft", B_force: Optional[int] = None,
-              transposed: bool = False) -> KernelPlan:
+              transposed: bool = False, live: int = 1) -> KernelPlan:
     """Plan for ``geom``.  ``need_lds``: the kernel exchanges a full transform through
     LDS after its passes (real-FFT post-processing), so reserve B padded rows.
     ``kind`` selects the tuned-plan entry (autotuner results / overrides) if any.
     ``transposed``: a plan of the transposed-kernel layout, whose order follows from the
-    threads and radices: these stay radix_plan's, so that stored kernels stay valid."""
+    threads and radices: these stay radix_plan's, so that stored kernels stay valid.
+    ``live``: sets of values a thread of a strided kernel holds at once."""
     twreg = False
     if radices is None:
         hit = lookup(geom, real, kind)
@@ -327,7 +334,10 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
                 if not dbl and wide * N * elem > LDS_BYTES_TARGET:
                     most = 16 if S * OUTER > 512 else 8 if S * OUTER > 64 else 4
                     wide = min(wide, most)
-                hit = column_radices(N, elem, wide)
+                hit = column_radices(N, elem, wide, live)
+                while hit is None and live > 1 and wide > 4:
+                    wide //= 2
+                    hit = column_radices(N, elem, wide, live)
                 if hit is not None:
                     radices, tt = hit
                     B_force = B_force or wide
@@ -411,6 +421,24 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
     return KernelPlan(real=real, N=N, TT=tt, B=B, S=S, OUTER=OUTER, radices=tuple(radices), COLFAST=colfast,
                       WAVE_LOCAL=wave_local, PAD_SHIFT=pad_shift, NP=NP, LDS_ELEMS=lds_elems, NWG=nwg,
                       NWG_INNER=nwg_inner, TWREG=twreg, LPW=lpw, CPAD=cpad)
+
+
+def roomier_plans(geom: AxisGeometry, real: str, kind: str, need_lds: bool = False) -> Iterator[KernelPlan]:
+    """Plans of fewer values a thread, for kernels that spill with the one they would have."""
+    N, plan = geom.N, None
+    radices, tt = ([N], 1) if geom.S > 1 and N <= 32 else radix_plan(N)
+    for how in (dict(kind=kind, live=2), dict(radices=radices, tt=tt, transposed=True)):
+        try:
+            plan = make_plan(geom, real, need_lds=need_lds, **how)
+        except ValueError:  # more threads or LDS than there are
+            continue
+        yield plan
+    if plan is not None and plan.CPAD:  # the padded addresses take registers, too
+        yield dataclasses.replace(plan, CPAD=False, LDS_ELEMS=plan.N * plan.B)
+
+
+def overridden(geom: AxisGeometry, real: str, kind: str) -> bool:
+    return plan_key(geom, real, kind) in _OVERRIDES
 
 
 def wave_bounds(plan: KernelPlan, conv: bool) -> Optional[Tuple[int, int]]:

@@ -13,7 +13,8 @@ from typing import Optional, Tuple
 from .. import dtypes as dt
 from . import hooks
 from .kernels import CompiledKernel, cfg_struct, kernel_symbol, translation_unit
-from .planner import AxisGeometry, KernelPlan, make_plan, transposed_size, wave_bounds, whole_xcds
+from .planner import (AxisGeometry, KernelPlan, make_plan, overridden, roomier_plans, transposed_size, wave_bounds,
+                      whole_xcds)
 from .precision import kernel_real_type
 
 
@@ -49,9 +50,17 @@ def _resolve_signal_range(signal_range, N: int) -> Tuple[int, int]:
     return s, e
 
 
-def conv_plan(buffer_shape, axis, compute_type, transposed: bool) -> KernelPlan:
+def conv_plan(buffer_shape, axis, compute_type, transposed: bool, live: int = 1) -> KernelPlan:
     geom = AxisGeometry.of(buffer_shape, axis)
-    return make_plan(geom, kernel_real_type(compute_type), kind="conv", transposed=transposed)
+    return make_plan(geom, kernel_real_type(compute_type), kind="conv", transposed=transposed, live=live)
+
+
+def with_roomier(build, plan: KernelPlan, geom: AxisGeometry, kind: str, need_lds: bool = False) -> CompiledKernel:
+    """``build(plan)``, which falls back to roomier plans if it turns out to spill."""
+    kernel = build(plan)
+    if not overridden(geom, plan.real, kind):
+        kernel.roomier = lambda: (build(p) for p in roomier_plans(geom, plan.real, kind, need_lds) if p != plan)
+    return kernel
 
 
 def _io_functors(args, output_map, input_map, output_type, input_type, compute, N, knum):
@@ -105,18 +114,21 @@ def make_fft_shader(buffer_shape: Tuple, axis: int = None, inverse: bool = False
     # share lines between neighbouring tiles: those tiles go to one XCD (one fetch)
     xcd = bool(input_map or output_map) or _unaligned((geom.S if geom.S > 1 else N) * output_type.item_size,
                                                       (geom.S if geom.S > 1 else N) * (input_type or output_type).item_size)
-    if xcd:
-        plan = whole_xcds(plan)
-    cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=N * geom.S, sig=sig, r2c=r2c, inverse=inverse,
-                     normalize=normalize, scale=1.0 / N, xcd_map=xcd)
     functors = _io_functors(args, output_map, input_map, output_type, input_type, compute, N, 1)
     kind = ("irfft" if inverse else "rfft") if r2c else "fft"
     tag = ("inv" if inverse else "fwd") + ("_hook" if (input_map or output_map) else "")
-    src = translation_unit(cfg, functors, "vkx::fft_body<Cfg, HookIn, HookOut>(prm);", plan.BLOCK,
-                           kernel_symbol(kind, plan, tag),
-                           None if input_map or output_map else wave_bounds(plan, False))
     name = f"fft_shader_{tuple(buffer_shape)}_{axis}_{inverse}_{normalize_inverse}_{r2c}"
-    return CompiledKernel(src, plan, args, list(plan.radices), None, name=name)
+
+    def build(plan):
+        if xcd:
+            plan = whole_xcds(plan)
+        cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=N * geom.S, sig=sig, r2c=r2c, inverse=inverse,
+                         normalize=normalize, scale=1.0 / N, xcd_map=xcd)
+        src = translation_unit(cfg, functors, "vkx::fft_body<Cfg, HookIn, HookOut>(prm);", plan.BLOCK,
+                               kernel_symbol(kind, plan, tag),
+                               None if input_map or output_map else wave_bounds(plan, False))
+        return CompiledKernel(src, plan, args, list(plan.radices), None, name=name)
+    return with_roomier(build, plan, geom, "fft")
 
 
 def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: bool, io_type, compute_type,
@@ -140,10 +152,6 @@ def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: 
     normalize = bool(inverse and normalize_inverse)
     # plain tile order: with the XCD-contiguous order the 1024-point rows of 513-value
     # spectra measured slower (67.1 / 57.2 against 61.6 / 54.2 us)
-    cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=0, sig=sig, r2c=True, inverse=inverse,
-                     normalize=normalize, scale=1.0 / N)
-    if packed:
-        cfg = cfg.replace("struct Cfg {", "struct Cfg {\n  static constexpr bool PACKED = true;", 1)
     from .hooks import Arg
     if oop:
         real_t = io_type.child_type
@@ -154,9 +162,16 @@ def _make_real_row_shader(geom: AxisGeometry, inverse: bool, normalize_inverse: 
     kind = "irfft" if inverse else "rfft"
     body = f"vkx::{kind}_body<Cfg, {io_type.child_type.cpp}, {'true' if oop else 'false'}>(prm);"
     tag = ("inv" if inverse else "fwd") + ("_oop" if oop else "") + ("_packed" if packed else "")
-    src = translation_unit(cfg, [], body, plan.BLOCK, kernel_symbol(kind + "h", plan, tag))
-    return CompiledKernel(src, plan, args, list(plan.radices), None, name=f"{kind}_shader_{geom.shape}",
-                          roots_n=N)
+
+    def build(plan):
+        cfg = cfg_struct(plan, in_os=in_os, out_os=out_os, k_os=0, sig=sig, r2c=True, inverse=inverse,
+                         normalize=normalize, scale=1.0 / N)
+        if packed:
+            cfg = cfg.replace("struct Cfg {", "struct Cfg {\n  static constexpr bool PACKED = true;", 1)
+        src = translation_unit(cfg, [], body, plan.BLOCK, kernel_symbol(kind + "h", plan, tag))
+        return CompiledKernel(src, plan, args, list(plan.radices), None, name=f"{kind}_shader_{geom.shape}",
+                              roots_n=N)
+    return with_roomier(build, plan, half_geom, kind, not inverse)
 
 
 @lru_cache(maxsize=None)
@@ -218,17 +233,12 @@ def make_convolution_shader(buffer_shape: Tuple, kernel_map=None, kernel_num: in
     compute = _compute_dtype(compute_type)
     geom = AxisGeometry.of(buffer_shape, axis)
     N = geom.N
-    plan = conv_plan(tuple(buffer_shape), axis, compute_type, transposed_kernel)
+    plan = conv_plan(tuple(buffer_shape), axis, compute_type, transposed_kernel, 2 if kernel_num > 1 else 1)
     args = hooks.declare_args(output_map, input_map, kernel_map, output_type, input_type, kernel_type, conv=True)
     k_args = [a for a in args if a.role == "kernel"]
     sig = _resolve_signal_range(input_signal_range, N)
     xcd = bool(input_map or output_map) or _unaligned(
         (geom.S if geom.S > 1 else N) * (output_type or compute_type).item_size)
-    if xcd and not transposed_kernel:
-        plan = whole_xcds(plan)
-    cfg = cfg_struct(plan, in_os=N * geom.S, out_os=N * geom.S, k_os=N * geom.S, sig=sig, r2c=False,
-                     inverse=False, normalize=bool(normalize), scale=1.0 / N, knum=kernel_num,
-                     k_inner_only=kernel_inner_only, k_transposed=transposed_kernel, xcd_map=xcd)
     functors = _io_functors(args, output_map, input_map, output_type, input_type, compute, N, kernel_num)
     if kernel_map is not None:
         functors.append(hooks.functor_source("HookKernel", kernel_map, k_args, compute, N, writing=False,
@@ -238,10 +248,20 @@ def make_convolution_shader(buffer_shape: Tuple, kernel_map=None, kernel_num: in
     tag = ("inner" if kernel_inner_only else "") + ("_t" if transposed_kernel else "") + \
         ("_hook" if (input_map or output_map or kernel_map) else "") + (f"_k{kernel_num}" if kernel_num > 1 else "")
     plain = not (input_map or output_map or kernel_map or transposed_kernel) and kernel_num == 1
-    src = translation_unit(cfg, functors, "vkx::conv_body<Cfg, HookIn, HookKernel, HookOut>(prm);", plan.BLOCK,
-                           kernel_symbol("conv", plan, tag), wave_bounds(plan, True) if plain else None)
-    return CompiledKernel(src, plan, args, list(plan.radices), list(reversed(plan.radices)),
-                          name=f"convolution_shader_{tuple(buffer_shape)}_{axis}")
+
+    def build(plan):
+        if xcd and not transposed_kernel:
+            plan = whole_xcds(plan)
+        cfg = cfg_struct(plan, in_os=N * geom.S, out_os=N * geom.S, k_os=N * geom.S, sig=sig, r2c=False,
+                         inverse=False, normalize=bool(normalize), scale=1.0 / N, knum=kernel_num,
+                         k_inner_only=kernel_inner_only, k_transposed=transposed_kernel, xcd_map=xcd)
+        src = translation_unit(cfg, functors, "vkx::conv_body<Cfg, HookIn, HookKernel, HookOut>(prm);", plan.BLOCK,
+                               kernel_symbol("conv", plan, tag), wave_bounds(plan, True) if plain else None)
+        return CompiledKernel(src, plan, args, list(plan.radices), list(reversed(plan.radices)),
+                              name=f"convolution_shader_{tuple(buffer_shape)}_{axis}")
+    if transposed_kernel:  # its layout follows from the plan
+        return build(plan)
+    return with_roomier(build, plan, geom, "conv")
 
 
 def get_cache_info():
