@@ -1,0 +1,39 @@
+"""Plans that depend on how much a launch has to do (fft/planner.py), on the CPU."""
+import numpy as np
+import pytest
+
+from vkdispatch_amd.fft import planner as P
+
+LENGTHS = [36, 45, 60, 96, 125, 143, 243, 338, 480, 500, 686, 720, 972, 1000, 1001, 1250, 2000, 2187, 4000]
+
+
+@pytest.mark.parametrize("real,elem", [("float", 8), ("double", 16)])
+@pytest.mark.parametrize("kind", ["fft", "conv", "rfft"])
+def test_plans_fit_at_every_size(real, elem, kind):
+    for n in LENGTHS:
+        for s in ((1,) if kind == "rfft" else (1, 32, 65, 257, 320)):
+            for outer in (1, 2, 17, 300, 5000):
+                try:
+                    p = P.make_plan(P.AxisGeometry((outer, n, s), 1, n, s, outer), real, kind=kind,
+                                    need_lds=kind == "rfft")
+                except ValueError:
+                    assert P.radix_plan(n)[1] > P.MAX_THREADS or n * elem > 128 * 1024
+                    continue
+                assert np.prod(p.radices) == n and p.BLOCK <= P.MAX_THREADS and p.lds_bytes <= P.LDS_BYTES_MAX
+                assert all(p.TT * -(-(n // r) // p.TT) >= n // r for r in p.radices)
+                assert p.NWG_INNER * p.B >= s if s > 1 else p.NWG * p.B >= outer
+                if kind == "rfft":
+                    assert p.LDS_ELEMS >= p.B * p.NP
+                if p.LPW:
+                    assert p.LPW * p.TT <= 64 and p.BLOCK // 64 * p.LPW == p.B
+
+
+def test_few_rows_and_many():
+    """Up to FEW_POINTS a row takes more threads and a workgroup one wave; complex128 and powers
+    of two are as they were."""
+    def rows(outer, n, real="float"):
+        return P.make_plan(P.AxisGeometry((outer, n), 1, n, 1, outer), real)
+    few, many = rows(P.FEW_POINTS // 500, 500), rows(P.FEW_POINTS // 500 + 1, 500)
+    assert few.VMAX <= 10 < many.VMAX and few.BLOCK == 64 < many.BLOCK
+    assert rows(1, 500, "double").radices == rows(5000, 500, "double").radices
+    assert rows(1, 512).radices == rows(5000, 512).radices
