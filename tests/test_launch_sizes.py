@@ -37,3 +37,14 @@ def test_few_rows_and_many():
     assert few.VMAX <= 10 < many.VMAX and few.BLOCK == 64 < many.BLOCK
     assert rows(1, 500, "double").radices == rows(5000, 500, "double").radices
     assert rows(1, 512).radices == rows(5000, 512).radices
+
+
+def test_few_tiles_and_many():
+    """Whole lines where the launch fills the chip several times over; narrower tiles where
+    it does not, or where the last round of large workgroups would be nearly empty."""
+    def cols(outer, n, s):
+        return P.make_plan(P.AxisGeometry.of((outer, n, s), 1), kind="conv")
+    assert cols(40, 1000, 257).B == 16 and cols(40, 1000, 320).B == 16
+    assert cols(2, 1000, 257).B < 16 and cols(16, 1000, 257).B < 16
+    assert cols(16, 1000, 257).NWG <= 256 * (P.LDS_BYTES_MAX // cols(16, 1000, 257).lds_bytes)
+    assert cols(40, 1000, 24).radices == cols(500, 1000, 24).radices  # strides it says nothing about

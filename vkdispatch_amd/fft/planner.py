@@ -166,6 +166,63 @@ def few_rows_plan(N: int, elem: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     return next(quick_radices(N, elem, 1.0), None)
 
 
+def column_time(N: int, S: int, OUTER: int, elem: int, conv: bool, B: int, radices, tt: int) -> float:
+    """Microseconds of a launch of strided transforms, B of them in a workgroup (fitted to 3264
+    launches of 25 lengths of 96 to 2000, strides of 64 to 513, 0.02 to 6 M points: 15 % rms):
+    rounds of workgroups times their own time, which is that of the values a thread handles
+    and of the barriers of its size, and the bytes at the rate of a CU and of the chip, more
+    of them where a tile is narrower than a cache line (much more where lines are not dealt to
+    the XCDs in whole rows of tiles, as for aligned strides)."""
+    held = [slots(N, r, tt) for r in radices]
+    passes = 2 if conv else 1
+    block = B * tt
+    registers = max(held) * (13 if elem == 16 else 7.2 if conv else 6) + 16
+    waves = max(1, min(8, int(512 // registers)), 4 if block > 768 else 3 if block > 512 else 2 if block > 256 else 1)
+    lds = (N + (N - 1) // radices[0]) * B * elem
+    side = max(1, min(LDS_BYTES_MAX // lds, 4 * waves // -(-block // WAVE), 2048 // block))
+    tiles = OUTER * -(-S // B)
+    each = -(-tiles // 256)
+    width = B * elem / 8
+    at4, at8 = (0.54, 0.23) if S * elem % 128 else (3.28, 1.07)
+    more = 0.0 if width >= 16 else at8 * (16 - width) / 8 if width >= 8 else \
+        at8 + (at4 - at8) * (8 - width) / 4 if width >= 4 else at4 * 4 / width
+    moved = each * 2 * min(B, S) * N * elem / 117e3 + 2 * OUTER * N * S * elem / 11.65e6
+    return 1.1 + -(-each // side) * (0.0615 * passes * sum(held) + 0.77 * block / 256) + moved * (1.0 + more)
+
+
+@lru_cache(maxsize=None)
+def column_plan(N: int, S: int, OUTER: int, elem: int, wide: int, conv: bool) -> Optional[Tuple[Tuple[int, ...], int, int]]:
+    """(radices, threads per transform, transforms per workgroup) of a strided launch: the tile
+    of ``wide`` transforms and its radices, or a narrower one, or fewer values a thread, where
+    column_time makes that much shorter (at strides like those it was fitted to).  Few tiles, or a
+    last round of large workgroups that is nearly empty, want more and smaller ones: 16 x 1000 x
+    257 transformed 26.3 -> 17.7 us, convolved 41.2 -> 25.9 (first-fit packing 19.1, 28.0); 2 x 1000
+    x 257 12.0 -> 6.5, 19.8 -> 9.0 (6.6, 9.1)."""
+    hit = column_radices(N, elem, wide)
+    if hit is None or S < 32:
+        return None if hit is None else (*hit, wide)
+    (rads, tt), dbl = hit, elem == 16
+    values, tiles = max(slots(N, r, tt) for r in rads), OUTER * -(-S // wide)
+    # sure gains only: the formula does not know how a kernel was scheduled, and many tiles
+    # leave less to gain (840 tiles of 252 points, predicted 0.85, took 1.11)
+    bounded = fewer_waves(dbl, conv, S, wide, tt, values, tiles, N * wide * elem) is not None
+    sure = 0.75 if bounded else 0.8 if tiles >= 512 else 0.9
+    best = (sure * column_time(N, S, OUTER, elem, conv, wide, rads, tt), rads, tt, wide)
+    quick = [(r[::-1], t) for (r, t), _ in zip(quick_radices(N, elem, 1.5), range(2))]
+    for B in [wide] + [w // elem for w in ((64, 48) if dbl else (64, 48, 32)) if w // elem < wide]:
+        hit = column_radices(N, elem, B)
+        for rads, tt in quick + ([hit] if hit else []):
+            values = max(slots(N, r, tt) for r in rads)
+            if B * tt > MAX_THREADS or (B * tt > 512 and values > (9 if dbl else 16)):
+                continue
+            if (N + (N - 1) // rads[0]) * B * elem > LDS_BYTES_MAX:
+                continue
+            time = column_time(N, S, OUTER, elem, conv, B, rads, tt)
+            if time < best[0]:
+                best = (time, rads, tt, B)
+    return best[1:]
+
+
 def radix_plan(N: int) -> Tuple[List[int], int]:
     """(radices, threads-per-transform) for a length-N transform done in one workgroup."""
     if N < 1:
@@ -364,13 +421,18 @@ def make_plan(geom: AxisGeometry, real: str = "float", batch_hint: Optional[int]
                 if not dbl and wide * N * elem > LDS_BYTES_TARGET:
                     most = 16 if S * OUTER > 512 else 8 if S * OUTER > 64 else 4
                     wide = min(wide, most)
-                hit = column_radices(N, elem, wide, live)
-                while hit is None and live > 1 and wide > 4:
-                    wide //= 2
+                if live == 1:
+                    hit = column_plan(N, S, OUTER, elem, wide, kind == "conv")
+                    if hit is not None:
+                        radices, tt, B_force = hit[0], hit[1], B_force or hit[2]
+                else:
                     hit = column_radices(N, elem, wide, live)
-                if hit is not None:
-                    radices, tt = hit
-                    B_force = B_force or wide
+                    while hit is None and wide > 4:
+                        wide //= 2
+                        hit = column_radices(N, elem, wide, live)
+                    if hit is not None:
+                        radices, tt = hit
+                        B_force = B_force or wide
             elif N > 32 and N not in _POW2 and tt <= MAX_THREADS:
                 few = OUTER * N <= FEW_POINTS and not dbl
                 hit = few_rows_plan(N, elem) if few else balanced_plan(N, elem)
@@ -486,16 +548,23 @@ def wave_bounds(plan: KernelPlan, conv: bool) -> Optional[Tuple[int, int]]:
     workgroups of 8 waves have a second one on the CU only with four waves: 28.7 -> 31.3),
     complex128 transforms with 15 and 16 (40 x 160 x 320 14.4 -> 12.3, none slower than 2 %);
     complex64 transforms lose 4 %."""
-    dbl = plan.real == "double"
-    if not plan.COLFAST or plan.S % plan.B or plan.TT == 1 or plan.BLOCK > 512 or plan.VMAX < (15 if dbl else 20):
+    if not plan.COLFAST:
         return None
-    least = -(-plan.BLOCK // (4 * WAVE))  # a workgroup's own
+    return fewer_waves(plan.real == "double", conv, plan.S, plan.B, plan.TT, plan.VMAX, plan.NWG, plan.LDS_ELEMS * 8)
+
+
+def fewer_waves(dbl: bool, conv: bool, S: int, B: int, tt: int, values: int, tiles: int,
+                lds: int) -> Optional[Tuple[int, int]]:
+    """wave_bounds of a strided plan."""
+    block = B * tt
+    if S % B or tt == 1 or block > 512 or values < (15 if dbl else 20):
+        return None
+    least = -(-block // (4 * WAVE))  # a workgroup's own
     if dbl:
         return None if conv else (least, 3)
-    if plan.NWG < 256:
+    if tiles < 256:
         return least, 2
-    lds = plan.LDS_ELEMS * 8
-    if conv and plan.BLOCK < 512 and (plan.VMAX >= 24 or (lds < 32 * 1024 and plan.BLOCK > WAVE)):
+    if conv and block < 512 and (values >= 24 or (lds < 32 * 1024 and block > WAVE)):
         return least, 3
     return None
 
