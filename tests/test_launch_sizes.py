@@ -48,3 +48,14 @@ def test_few_tiles_and_many():
     assert cols(2, 1000, 257).B < 16 and cols(16, 1000, 257).B < 16
     assert cols(16, 1000, 257).NWG <= 256 * (P.LDS_BYTES_MAX // cols(16, 1000, 257).lds_bytes)
     assert cols(40, 1000, 24).radices == cols(500, 1000, 24).radices  # strides it says nothing about
+
+
+def test_which_batches_of_small_images_take_one_launch():
+    """Beyond two images to a CU, only sizes whose workgroups keep it busy."""
+    from vkdispatch_amd.fft import half2d
+    def pays(n, h, w):
+        return half2d.whole_pays(n, h, w // 2)
+    assert all(pays(n, h, w) for n in (96, 256, 512) for h, w in ((96, 96), (128, 128), (60, 100), (200, 100)))
+    assert all(pays(n, h, w) for n in (600, 1024) for h, w in ((32, 32), (48, 96), (64, 128), (128, 128), (16, 1000)))
+    assert not any(pays(n, h, w) for n in (800, 1024) for h, w in ((96, 96), (60, 100), (96, 120), (128, 96)))
+    assert not pays(95, 128, 128) and pays(1, 64, 64) and not pays(1024, 160, 200)

@@ -149,14 +149,34 @@ def whole_plan(h: int, m: int):
     return rows, cols, min(shared or pitches, key=lambda p: (_bank_conflicts(h, m, rows, cols, p), p))
 
 
+def _waves(h: int, m: int, row_threads: int, column_threads: int) -> int:
+    """Waves of a workgroup that holds an h x 2m image: one for the lines of each."""
+    return min(WHOLE_WAVES, max(-(-h // (64 // row_threads)), -(-m // (64 // column_threads))))
+
+
 def whole_pays(images: int, h: int, m: int) -> bool:
     """Whether one workgroup per image beats three launches over all of them.  128^2: 256
     images 19.3 against 37.3 us, 96 17.9 / 19.5, 64 17.5 / 16.0 (the image alone takes 16.6, as
     long as one CU computes); 64^2: 1024 images 16.6 / 37, 4 images 8.2 / 10.  An image
     that leaves room for no second workgroup and few waves (160 x 200: 131 KB) is slower at
-    any count."""
+    any count.  From 513 images on a CU takes three and more of them in turn, while three launches
+    gain on larger batches: 1024 images of 96^2 67 / 54 us, 800 of 96 x 120 67.5 / 56.5, but of
+    128^2 68 / 79, of 64 x 128 28 / 47 (24 sizes, 12 counts of 96 to 1024)."""
     plan = whole_plan(h, m)
-    return plan is not None and 8 * h * plan[2] <= WHOLE_LDS and (images >= 96 or h * m <= 4096)
+    if plan is None or 8 * h * plan[2] > WHOLE_LDS or (images < 96 and h * m > 4096):
+        return False
+    (rr, rtt), (cr, ctt), pitch = plan
+    waves = _waves(h, m, rtt, ctt)
+    side = min(LDS_BYTES_MAX // (8 * (h * pitch + 2 * (h + m) + m)), 32 // waves)
+    if images <= 512 or h * m <= 2400 or side <= 1:
+        return True
+    # lines of a wave times the values of a thread, over the waves that a CU has at work on its
+    # four SIMDs (5 and 6 waves of an image leave some of them idle)
+    work = 2 * (-(-h // (64 // rtt)) * sum(slots(m, r, rtt) for r in rr) +
+                -(-m // (64 // ctt)) * sum(slots(h, r, ctt) for r in cr))
+    busy = min(32, waves * side) * waves / (4 * -(-waves // 4))
+    points = images * h * 2 * m / 1e6
+    return 4 + -(-images // 256) * 0.36 * work / busy < 1.05 * max(min(13 + 6.2 * points, 41), 5.3 * points)
 
 
 class HalfWhole:
@@ -165,8 +185,7 @@ class HalfWhole:
 
     def __init__(self, images: int, h: int, m: int, kstep: int, normalize: bool):
         (rr, rtt), (cr, ctt), pitch = whole_plan(h, m)
-        waves = min(WHOLE_WAVES, max(-(-h // (64 // rtt)), -(-m // (64 // ctt))))
-        block = 64 * waves
+        block = 64 * _waves(h, m, rtt, ctt)
         pl = lambda rs: "vkx::PL<" + ", ".join(f"vkx::P<{r}, {ns}>" for r, ns in pass_list(rs)) + ">"  # noqa: E731
 
         def line(name, n, radices, tt):

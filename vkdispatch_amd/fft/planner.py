@@ -161,8 +161,10 @@ FEW_POINTS = 1 << 19  # of a launch of rows; twice as many fill every SIMD
 def few_rows_plan(N: int, elem: int) -> Optional[Tuple[Tuple[int, ...], int]]:
     """(radices, threads) of launches of at most FEW_POINTS: three passes of up to 10 values
     rather than two of up to 32, one wave a workgroup.  25 lengths of 96 to 2000 points, real and
-    complex, 2^14 to 2^19 points, against balanced_plan: 0.78 to 0.86 of the time (500 real points,
-    524 rows, 7.1 -> 3.8 us; first-fit packing 4.7); at 2^20 0.92, some lengths slower."""
+    complex, 2^14 to 2^19 points, against balanced_plan: 0.78 to 0.86 of the time (524 x 500 real
+    points 7.1 -> 4.3 us, first-fit packing 5.1; 262 x 1000 complex 5.0 -> 3.8, 4.5); at 2^20 0.92,
+    some lengths slower.  261 launches of random sizes: 68 took over 5 % more than with
+    first-fit packing, 12 do."""
     return next(quick_radices(N, elem, 1.0), None)
 
 
@@ -196,8 +198,9 @@ def column_plan(N: int, S: int, OUTER: int, elem: int, wide: int, conv: bool) ->
     of ``wide`` transforms and its radices, or a narrower one, or fewer values a thread, where
     column_time makes that much shorter (at strides like those it was fitted to).  Few tiles, or a
     last round of large workgroups that is nearly empty, want more and smaller ones: 16 x 1000 x
-    257 transformed 26.3 -> 17.7 us, convolved 41.2 -> 25.9 (first-fit packing 19.1, 28.0); 2 x 1000
-    x 257 12.0 -> 6.5, 19.8 -> 9.0 (6.6, 9.1)."""
+    257 transformed 26.2 -> 18.7 us, convolved 40.5 -> 27.8 (first-fit packing 19.2, 27.8); 2 x 1000
+    x 257 11.9 -> 6.4, 19.6 -> 9.0 (6.6, 9.1).  417 launches of random sizes: 64 took over 5 % more
+    than with first-fit packing, 23 do (complex128 8 x 972 x 257 20.0 us, 15.0, among them)."""
     hit = column_radices(N, elem, wide)
     if hit is None or S < 32:
         return None if hit is None else (*hit, wide)
