@@ -292,3 +292,55 @@ def test_plans_on_one_stream_share_a_buffer(device, monkeypatch):
     monkeypatch.setattr(scratch, "_pinned", [])
     scratch.clear()
     assert not scratch._streams and len(device.freed) == 21
+
+
+def test_lengths_of_the_ragged_executor(device, monkeypatch):
+    """Prime factors above 13: a plan for each stream's calls and for each graph, whose launches
+    share it; a capture, which cannot build one, takes the newest."""
+    from vkdispatch_amd.fft import ragged
+    made, ran = [], []
+
+    class Plan:
+        n_items = 3
+
+        def __init__(self, sizes, **kw):
+            assert sizes == [20011] * 3
+            made.append(self)
+
+        def bind(self, buf):
+            return lambda stream=None: ran.append((self, device.stream if stream is None else stream))
+
+        def __call__(self, buf):
+            self.bind(buf)()
+    monkeypatch.setattr(ragged, "RaggedFFT", Plan)
+    monkeypatch.setattr(F, "_RAGGED_PLANS", {})
+    monkeypatch.setattr(scratch, "_pinned", [])
+
+    def call(graph=None):
+        assert F._large_or_prime_fallback((_Data(100),), (3, 20011), None, False, True, False, None, None, dt.complex64,
+                                          dt.complex64, None, graph)
+    for device.stream in (1, 5, 1):
+        call()
+    device.stream = 1
+    graphs = [G.CommandGraph(), G.CommandGraph()]
+    for g in graphs:
+        call(g)
+        call(g)
+    assert len(made) == 4
+    for g, s in zip(graphs, (7, 8)):
+        g._replay(s)
+    owners = {}
+    for plan, s in ran:
+        owners.setdefault(s, set()).add(plan)
+    assert sorted(owners) == [1, 5, 7, 8] and all(len(p) == 1 for p in owners.values())
+    assert len(set.union(*owners.values())) == 4
+    device.stream, device.capturing = 9, {9: 1}
+    call()
+    assert len(made) == 4 and ran[-1] == (made[0], 9)  # stream 1 called last
+    graphs[0].submit(stream=9)
+    assert scratch._pinned == [made[0], made[2]]  # what was captured is kept,
+    device.capturing = {}
+    for device.stream in range(20, 30):
+        call()
+    (calls,) = F._RAGGED_PLANS.values()
+    assert len(calls) == scratch.SCRATCH_STREAMS and made[0] not in calls.values()  # also when no call has it any more

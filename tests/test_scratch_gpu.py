@@ -102,3 +102,28 @@ def test_convolutions_on_two_streams():
         torch.cuda.synchronize()
         for b, ref in zip(bufs, refs):
             assert_close(b.read_real(0), ref, rel=1e-5)
+
+
+@pytest.mark.parametrize("count", [3, 24])
+def test_prime_lengths_on_two_streams(count):
+    """The ragged executor's lengths: items of the persistent kernel (3), a length class on side
+    streams (24)."""
+    print("scratch: prime lengths on two streams", count, flush=True)
+    rng = np.random.default_rng(count)
+    xs = [crand(rng, (count, 20011)) for _ in range(3)]
+    refs = [np.fft.fft(x.astype(np.complex128), axis=1) for x in xs]
+    bufs = [vd.asbuffer(x) for x in xs]
+    g = vd.CommandGraph()
+    vd.fft.fft(bufs[2], graph=g)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for _ in range(3):
+        for b, x in zip(bufs, xs):
+            b.write(x)
+        vd.synchronize()
+        g.submit(stream=streams[2].cuda_stream)
+        for s, b in zip(streams, bufs[:2]):
+            with vd.stream_scope(s):
+                vd.fft.fft(b)
+        torch.cuda.synchronize()
+        for b, ref in zip(bufs, refs):
+            assert_close(b.read(0), ref, rel=1e-5)

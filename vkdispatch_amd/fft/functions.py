@@ -174,44 +174,72 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
             or out_t is not dt.complex64 or comp_t not in (dt.complex64, dt.complex32)):
         return False
     from .long import LongFFT
-    plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize))
+    from .scratch import launch_order
+    record = graph is not None and not graph.submit_on_record
+    plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize), graph if record else None)
     buf = buffers[0]
-    if graph is not None and not graph.submit_on_record:
-        if isinstance(plan, LongFFT):
-            plan.record(buf, graph)
-        else:
-            graph.record_callable(plan.bind(buf))
+    if not record:
+        with launch_order():
+            plan(buf)
+    elif isinstance(plan, LongFFT):
+        plan.record(buf, graph)
     else:
-        plan(buf)
+        graph.record_callable(plan.bind(buf))
     return True
 
 
-def _uniform_plan(n, count, inverse, normalize):
+def _uniform_plan(n, count, inverse, normalize, graph=None):
     from . import long
-    from .ragged import RaggedFFT
     key = (n, count, inverse, normalize)
-    if key not in _UNIFORM_PLANS:
-        if long.split_length(n) is not None:
-            try:
-                _UNIFORM_PLANS[key] = long.LongFFT(n, count, inverse, normalize)
-                return _UNIFORM_PLANS[key]
-            except SpillError:  # a radix list whose kernel does not fit the registers
-                pass
+    if key in _LONG_PLANS:
+        return _LONG_PLANS[key]
+    if long.split_length(n) is not None and key not in _RAGGED_PLANS:
+        try:
+            _LONG_PLANS[key] = long.LongFFT(n, count, inverse, normalize)
+            return _LONG_PLANS[key]
+        except SpillError:  # a radix list whose kernel does not fit the registers
+            pass
+    return _ragged_plan(key, graph)
+
+
+def _ragged_plan(key, graph):
+    """A ragged plan's launches share its counters and scratch, so calls on different streams,
+    and every graph, have plans of their own (those of the last SCRATCH_STREAMS streams are
+    kept).  Inside a capture of the caller's, which cannot allocate, the newest one is
+    taken: its replays must not overlap with calls that have it."""
+    from .. import runtime as rt
+    from .ragged import RaggedFFT
+    from .scratch import SCRATCH_STREAMS, pin
+    capturing = rt.is_capturing()
+    calls = _RAGGED_PLANS.setdefault(key, {})
+    kept, owner = (calls, rt.stream_key(rt.current_stream())) if graph is None else (graph.plans, key)
+    plan = kept.pop(owner, None)
+    if plan is None:
+        if calls and capturing:
+            pin(next(reversed(calls.values())))
+            return next(reversed(calls.values()))
+        n, count, inverse, normalize = key
         plan = RaggedFFT([n] * count, inverse=inverse, normalize=normalize, block=512)
         if plan.n_items > count and count > 128:
             # many tiled transforms: 256-thread workgroups (65536 x 256 points: 298 vs
             # 371 us); whole transforms and small tiled batches run faster at 512
             plan.block = plan.block_first = 256
-        _UNIFORM_PLANS[key] = plan
-    return _UNIFORM_PLANS[key]
+    if capturing:
+        pin(plan)
+    kept[owner] = plan  # the newest comes last
+    while len(calls) > SCRATCH_STREAMS:
+        del calls[next(iter(calls))]
+    return plan
 
 
-_UNIFORM_PLANS: dict = {}
+_LONG_PLANS: dict = {}
+_RAGGED_PLANS: dict = {}
 
 
 def _clear_uniform_plans() -> None:
     from . import long
-    _UNIFORM_PLANS.clear()
+    _LONG_PLANS.clear()
+    _RAGGED_PLANS.clear()
     long.clear()
 
 

@@ -39,6 +39,12 @@ def launch_order():
     return _order
 
 
+def pin(owner) -> None:
+    """Keep what a capture of the caller's launches with, whatever drops it, until clear()."""
+    if not any(o is owner for o in _pinned):
+        _pinned.append(owner)
+
+
 class StreamScratch:
     """Owner of launches with ``_points`` complex64 values between them."""
 
@@ -73,8 +79,7 @@ class StreamScratch:
             full = len(kept) >= SCRATCH_CAPTURES
             oldest = next((k for k in kept if k[2] >= self._points), None) if full else None
             kept[key] = self._new_scratch() if oldest is None else kept.pop(oldest)
-            if self not in _pinned:
-                _pinned.append(self)  # a plan cache may drop the plan; the captured graph needs its memory
+            pin(self)
         return kept[key]
 
 

@@ -25,6 +25,7 @@ class CommandGraph:
         # (kernel or launcher, device pointers, packed constants, objects kept alive)
         self._records: List[Tuple[object, Optional[List[int]], Optional[bytes], tuple]] = []
         self._scratch = None  # StreamScratch of the records that need one
+        self.plans: dict = {}  # plans that only launches recorded here use, one after another
         self._exec: Optional[int] = None
         self._exec_stream = None
         self._exec_scratch = None
@@ -116,6 +117,10 @@ class CommandGraph:
         if cap is not None or rt.is_capturing(s):
             # the caller is capturing this stream (torch.cuda.graph): launch the records
             # directly so that they become nodes of the caller's graph
+            if self.plans:
+                from .fft.scratch import pin
+                for plan in self.plans.values():
+                    pin(plan)
             for _ in range(reps):
                 self._replay_now(s)
         elif use_graph:
@@ -132,6 +137,7 @@ class CommandGraph:
         self._drop_exec()
         self._records = []
         self._scratch = None
+        self.plans = {}
 
     def destroy(self) -> None:
         self.reset()
