@@ -20,13 +20,16 @@ from functools import lru_cache
 from typing import List, NamedTuple, Optional, Tuple, Union
 
 from .. import dtypes as dt
+from .. import runtime as rt
 from ..buffer import Buffer, RFFTBuffer
 from ..graph import CommandGraph, dispatch
 from ..shader_map import MappingFunction
+from . import long
 from . import precision as prec
 from .kernels import SpillError
 from .shader_factories import (get_transposed_size, make_convolution_shader, make_fft_shader,
                                make_transpose_shader, register_plan_cache)
+from .scratch import SCRATCH_STREAMS, launch_order, pin
 
 
 def _validate_map_argument_annotations(map_fn: MappingFunction, map_name: str) -> None:
@@ -173,15 +176,13 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
     if (geom.S != 1 or r2c or input_map is not None or output_map is not None or signal_range is not None
             or out_t is not dt.complex64 or comp_t not in (dt.complex64, dt.complex32)):
         return False
-    from .long import LongFFT
-    from .scratch import launch_order
     record = graph is not None and not graph.submit_on_record
     plan = _uniform_plan(geom.N, geom.OUTER, bool(inverse), bool(normalize), graph if record else None)
     buf = buffers[0]
     if not record:
         with launch_order():
             plan(buf)
-    elif isinstance(plan, LongFFT):
+    elif isinstance(plan, long.LongFFT):
         plan.record(buf, graph)
     else:
         graph.record_callable(plan.bind(buf))
@@ -189,17 +190,14 @@ def _large_or_prime_fallback(buffers, buffer_shape, axis, inverse, normalize, r2
 
 
 def _uniform_plan(n, count, inverse, normalize, graph=None):
-    from . import long
     key = (n, count, inverse, normalize)
-    if key in _LONG_PLANS:
-        return _LONG_PLANS[key]
-    if long.split_length(n) is not None and key not in _RAGGED_PLANS:
+    plan = _LONG_PLANS.get(key)
+    if plan is None and key not in _RAGGED_PLANS and long.split_length(n) is not None:
         try:
-            _LONG_PLANS[key] = long.LongFFT(n, count, inverse, normalize)
-            return _LONG_PLANS[key]
+            plan = _LONG_PLANS[key] = long.LongFFT(n, count, inverse, normalize)
         except SpillError:  # a radix list whose kernel does not fit the registers
             pass
-    return _ragged_plan(key, graph)
+    return _ragged_plan(key, graph) if plan is None else plan
 
 
 def _ragged_plan(key, graph):
@@ -207,9 +205,6 @@ def _ragged_plan(key, graph):
     and every graph, have plans of their own (those of the last SCRATCH_STREAMS streams are
     kept).  Inside a capture of the caller's, which cannot allocate, the newest one is
     taken: its replays must not overlap with calls that have it."""
-    from .. import runtime as rt
-    from .ragged import RaggedFFT
-    from .scratch import SCRATCH_STREAMS, pin
     capturing = rt.is_capturing()
     calls = _RAGGED_PLANS.setdefault(key, {})
     kept, owner = (calls, rt.stream_key(rt.current_stream())) if graph is None else (graph.plans, key)
@@ -218,6 +213,7 @@ def _ragged_plan(key, graph):
         if calls and capturing:
             pin(next(reversed(calls.values())))
             return next(reversed(calls.values()))
+        from .ragged import RaggedFFT
         n, count, inverse, normalize = key
         plan = RaggedFFT([n] * count, inverse=inverse, normalize=normalize, block=512)
         if plan.n_items > count and count > 128:
@@ -237,7 +233,6 @@ _RAGGED_PLANS: dict = {}
 
 
 def _clear_uniform_plans() -> None:
-    from . import long
     _LONG_PLANS.clear()
     _RAGGED_PLANS.clear()
     long.clear()

@@ -15,11 +15,10 @@ from __future__ import annotations
 
 import os
 from functools import lru_cache
-from typing import Dict, List, Optional, Sequence, Tuple
+from typing import Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 from .. import dtypes as dt
 from .. import runtime as rt
-from ..buffer import Buffer
 from ..graph import CommandGraph, dispatch
 from . import half2d
 from .hooks import Arg
@@ -93,6 +92,11 @@ def _conv_tu(cfg: str, symbol: str, block: int, waves_per_simd: Optional[int], b
                       f"  {body}", "}", ""])
 
 
+class _Address(NamedTuple):
+    """A place in a buffer that is passed as well."""
+    ptr: int
+
+
 class Conv2DPhases(StreamScratch):
     """The same computation as three ordinary kernels in stream order: row FFTs of the
     image pairs (plus the kernel prep), column FFT * Kt * IFFT, row IFFTs; each pair's
@@ -148,8 +152,7 @@ class Conv2DPhases(StreamScratch):
             _check_no_spill(self.kernels())
             self._checked = True
         scr = self._scratch_for(rt.current_stream()) if scratch is None else scratch
-        kt = Buffer((self.H, self.W), dt.complex64, external=(scr.ptr + 8 * self.npairs * self.H * self.W, scr, True))
-        return [buffer, kernel, scr, scr, scr, kt]
+        return [buffer, kernel, scr, scr, scr, _Address(scr.ptr + 8 * self.npairs * self.H * self.W)]
 
     def __call__(self, buffer, kernel, graph=None) -> None:
         if isinstance(graph, CommandGraph) and not graph.submit_on_record:

@@ -315,8 +315,9 @@ def _raise_async_errors(stream: int) -> None:
 def is_capturing(stream=None) -> bool:
     """True while ``stream`` (default: the current stream) is being captured into a graph."""
     c = ctypes.c_int(0)
-    check(lib().vkx_stream_is_capturing(current_stream() if stream is None else int(stream), ctypes.byref(c)),
-          "vkx_stream_is_capturing")
+    rc = lib().vkx_stream_is_capturing(current_stream() if stream is None else int(stream), ctypes.byref(c))
+    if rc:
+        check(rc, "vkx_stream_is_capturing")
     return c.value != 0
 
 
