@@ -344,3 +344,28 @@ def test_lengths_of_the_ragged_executor(device, monkeypatch):
         call()
     (calls,) = F._RAGGED_PLANS.values()
     assert len(calls) == scratch.SCRATCH_STREAMS and made[0] not in calls.values()  # also when no call has it any more
+
+
+def test_a_graph_waits_for_a_call_to_be_enqueued(device, monkeypatch):
+    """A thread submits a graph on the stream of a call that is between its launches."""
+    monkeypatch.setattr(scratch, "_streams", {})
+    plan, log, call, _ = _long(monkeypatch)
+    graph = G.CommandGraph()
+    call(_Data(1 << 25), graph)
+    graph.capture(1)
+    del log[:]
+    device.vkx_graph_launch = lambda ex, s: log.append(("graph", s, ())) or 0
+    inside, other = threading.Event(), threading.Event()
+
+    class Slow(_Kernel):
+        def launch_raw(self, ptrs, consts=b"", stream=None):
+            super().launch_raw(ptrs, consts, stream)
+            if not inside.is_set():
+                inside.set()
+                other.wait(0.3)
+    plan.kernels = {c: (Slow(log, "cols"), plan.kernels[c][1]) for c in (1, 2)}
+    t = threading.Thread(target=lambda: (inside.wait(), graph.submit(stream=1), other.set()))
+    t.start()
+    call(_Data(1 << 26), None)
+    t.join()
+    assert [n for n, _, _ in log] in (["cols", "rows"] * 2 + ["graph"], ["graph"] + ["cols", "rows"] * 2)

@@ -83,12 +83,15 @@ class CommandGraph:
             else:
                 k.launch_raw(ptrs, consts, stream)
 
-    def _replay_now(self, stream: int) -> None:
+    def _order(self):
+        """Held while launches that use a stream's scratch are enqueued (fft/scratch.py)."""
         if self._scratch is None:
-            self._replay(stream)
-            return
+            return contextlib.nullcontext()
         from .fft.scratch import launch_order
-        with launch_order():
+        return launch_order()
+
+    def _replay_now(self, stream: int) -> None:
+        with self._order():
             self._replay(stream, self._scratch_on(stream))
 
     def capture(self, stream: Optional[int] = None) -> int:
@@ -124,9 +127,10 @@ class CommandGraph:
             for _ in range(reps):
                 self._replay_now(s)
         elif use_graph:
-            ex = self.capture(s)
-            for _ in range(reps):
-                rt.check(rt.lib().vkx_graph_launch(ex, s), "vkx_graph_launch")
+            with self._order():
+                ex = self.capture(s)
+                for _ in range(reps):
+                    rt.check(rt.lib().vkx_graph_launch(ex, s), "vkx_graph_launch")
         else:
             for _ in range(reps):
                 self._replay_now(s)
