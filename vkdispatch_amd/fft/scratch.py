@@ -62,13 +62,15 @@ class StreamScratch:
         with self._lock:
             if rt.is_capturing(stream):
                 return self._scratch_of_capture(stream)
-            key = rt.stream_key(stream)
-            have = self._scratch.pop(key, None)
-            if have is None or have[0] < self._points:
-                have = (self._points, self._new_scratch())
-            self._scratch[key] = have  # the newest comes last
-            while len(self._scratch) > SCRATCH_STREAMS:
-                del self._scratch[next(iter(self._scratch))]
+            kept, key = self._scratch, rt.stream_key(stream)
+            have = kept.get(key)
+            if have is None or have[0] < self._points or next(reversed(kept)) != key:
+                kept.pop(key, None)
+                if have is None or have[0] < self._points:
+                    have = (self._points, self._new_scratch())
+                kept[key] = have  # the newest comes last
+                while len(kept) > SCRATCH_STREAMS:
+                    del kept[next(iter(kept))]
             return have[1]
 
     def _scratch_of_capture(self, stream: int):

@@ -176,6 +176,10 @@ class _State(threading.local):
     stream_override = None
     allocating_in_capture = False
 
+    def __init__(self):
+        self.flag = ctypes.c_int(0)  # of is_capturing
+        self.flag_ref = ctypes.byref(self.flag)
+
 
 _state = _State()
 _device_lock = threading.Lock()
@@ -314,11 +318,10 @@ def _raise_async_errors(stream: int) -> None:
 
 def is_capturing(stream=None) -> bool:
     """True while ``stream`` (default: the current stream) is being captured into a graph."""
-    c = ctypes.c_int(0)
-    rc = lib().vkx_stream_is_capturing(current_stream() if stream is None else int(stream), ctypes.byref(c))
+    rc = (_lib or lib()).vkx_stream_is_capturing(current_stream() if stream is None else stream, _state.flag_ref)
     if rc:
         check(rc, "vkx_stream_is_capturing")
-    return c.value != 0
+    return _state.flag.value != 0
 
 
 def stream_key(stream: int):
