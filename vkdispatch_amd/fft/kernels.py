@@ -397,11 +397,11 @@ class SpillError(RuntimeError):
 
 
 def check_no_spill(kernel: "CompiledKernel") -> None:
-    """Refuse a kernel whose code object spills registers to private memory.  Every
-    kernel the planners emit is built to stay in registers (the tuned plans, the
-    pair-packed convolutions and every FFT shape of the test suite compile without
-    spills); a spilling variant once produced wrong rows on the MI355X with no cause
-    found, so a plan that spills is an error here, never a silent slow path."""
+    """Refuse a kernel whose code object needs private memory.  Kernels are built to stay
+    in registers, and one that does not has been replaced by a roomier plan's before it
+    comes here (CompiledKernel.settle); what is left are plans that were asked for by their
+    numbers and launches for which no plan fits.  A spilling variant once produced wrong
+    rows on the MI355X with no cause found, so it is an error, never a silent slow path."""
     info = kernel.code_object_info()
     if info["private_bytes"]:
         raise SpillError(f"{kernel.name}: {info['private_bytes']} bytes/lane of register spills "
